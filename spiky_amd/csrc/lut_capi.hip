@@ -332,6 +332,11 @@ hipError_t layout_propagate_tm(const spiky::FcShape &s, spiky::Scratch &x) {
                                       nullptr);
 }
 
+hipError_t layout_propagate_fc(const spiky_lut_manager *m, const spiky::FcShape &s, spiky::Scratch &x) {
+    return spiky::launch_propagate_fc(s, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                      m->int_mode, m->int_rescaler, x, nullptr);
+}
+
 hipError_t layout_wgrad_fc(const spiky_lut_manager *m, const spiky::FcShape &s, spiky::Scratch &x) {
     return spiky::launch_wgrad_fc(s, nullptr, nullptr, nullptr, 1.0, m->int_mode, m->int_rescaler, true, x,
                                   nullptr);
@@ -376,7 +381,7 @@ hipError_t layout_backward_product(const spiky_lut_manager *m, const spiky::Prod
 }
 
 // The fully connected backward's one scratch buffer, used in stream order:
-// the table-major propagate's layout first, then the weight gradient's (whose
+// the propagate's layout first, then the weight gradient's (whose
 // bucket sort reads the transposed keys the propagate leaves at the start of
 // its region).
 struct FcBackwardRegions {
@@ -388,9 +393,9 @@ struct FcBackwardRegions {
 FcBackwardRegions fc_backward_regions(const spiky_lut_manager *m, const spiky::FcShape &s, bool with_wgrad) {
     FcBackwardRegions r;
     r.tm = !m->int_mode && spiky::tm_propagate_applies(s);
-    if (r.tm)
-        r.prop_bytes = align256(planned_bytes([&](spiky::Scratch &x) { return layout_propagate_tm(s, x); },
-                                              "propagate_through_detectors_fc"));
+    r.prop_bytes = align256(planned_bytes(
+        [&](spiky::Scratch &x) { return r.tm ? layout_propagate_tm(s, x) : layout_propagate_fc(m, s, x); },
+        "propagate_through_detectors_fc"));
     if (with_wgrad)
         r.wg_bytes = planned_bytes([&](spiky::Scratch &x) { return layout_wgrad_fc(m, s, x); },
                                    "gather_w_gradients_fc");
@@ -846,15 +851,12 @@ int spiky_lut_backward_backprop(spiky_lut_manager *m, float *weights, uint32_t b
                                                             input_grad, prop_scr, st),
                                  "propagate_through_detectors_fc");
                 else
-                    check_hip(spiky::launch_propagate_fc(s, weights, output_grad, lookup_indices,
-                                                         min_deltas, min_delta_indices, anchors,
-                                                         input_grad, m->int_mode, m->int_rescaler, st),
-                              "propagate_through_detectors_fc");
+                    check_launch(spiky::launch_propagate_fc(s, weights, output_grad, lookup_indices,
+                                                            min_deltas, min_delta_indices, anchors,
+                                                            input_grad, m->int_mode, m->int_rescaler,
+                                                            prop_scr, st),
+                                 "propagate_through_detectors_fc");
             });
-            if (m->int_mode)
-                check_hip(spiky::launch_convert_i2f(input_grad, (uint64_t)batch_size * m->n_inputs,
-                                                    m->int_rescaler, st),
-                          "convert_integers_to_floats");
             if (target) {
                 m->timed("gather_w_gradients_fc", st, [&] {
                     // the table-major propagate left the transposed keys at its scratch start
@@ -1347,9 +1349,9 @@ int spiky_lut_scratch_plan(spiky_lut_manager *m, int op, uint32_t batch_size, ui
                 if (fc) {
                     const FcBackwardRegions r = fc_backward_regions(m, s, wg);
                     *needed = r.prop_bytes + r.wg_bytes;
-                    if (r.tm)
-                        check_region([&](spiky::Scratch &x) { return layout_propagate_tm(s, x); }, 0, r.prop_bytes,
-                                     "propagate_through_detectors_fc");
+                    check_region(
+                        [&](spiky::Scratch &x) { return r.tm ? layout_propagate_tm(s, x) : layout_propagate_fc(m, s, x); },
+                        0, r.prop_bytes, "propagate_through_detectors_fc");
                     if (wg)
                         check_region([&](spiky::Scratch &x) { return layout_wgrad_fc(m, s, x); }, r.prop_bytes,
                                      UINT64_MAX, "gather_w_gradients_fc");

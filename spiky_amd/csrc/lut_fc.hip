@@ -18,14 +18,13 @@
 //                       tables and an fp32 (or int32) running sum -- the exact
 //                       commit order of the reference CPU path, so the output is
 //                       bit-identical to it.
-//   k_propagate_fc_fast one wavefront per (sample, chunk of tables); chunks are
-//                       mapped to XCDs; coalesced float4 reads of the main and
-//                       the flipped row, fp64 dot, one pair of fp32 atomics per
-//                       (sample, table).
+//   k_propagate_rows    one wavefront per (few samples, run of tables); a lane
+//                       owns a 32-output block of a (sample, table) item, fed
+//                       from coalesced row reads through LDS, and sums it in
+//                       fp64 in output order (both summations).
 //   k_propagate_fc_exact one thread per (b, t, output block): the reference's
-//                       own decomposition, used for int32 summation (its
-//                       payloads must be formed per block to stay bit-exact) and
-//                       for shapes the fast kernel does not cover.
+//                       own decomposition, for int32 payloads of other block
+//                       sizes and for very small calls.
 //   k_bucket_samples +  table-major weight gradient: a stable counting sort of
 //   k_wgrad_rowsum      the samples of every table by lookup index, then one
 //                       wavefront per table row summing g over its bucket in
@@ -449,95 +448,228 @@ __global__ __launch_bounds__(kBlock) void k_propagate_fc_exact(
 }
 
 // ---------------------------------------------------------------------------
-// propagate, fp32-summation form over column slices.  Wavefront = SPW samples
-// x one column slice (slice -> XCD as in the forward).  For every (sample,
-// table) the lane-partial fp64 dot  sum_c (W_main[c] - W_alt[c]) * g[c]  over
-// the slice is reduced across the wavefront, scaled by du(min margin), and
-// committed as one pair of fp32 atomics per (sample, table, slice).  The
-// reference commits one pair per 32-output block (forward_group_size); the
-// slice commit differs from it only in fp32 rounding of the committed terms.
+// The same gradient over gathered rows (both summations).  A unit is one
+// 32-output block of one (sample, table) item, and a lane owns a unit: it sums
+// its block of the main and the flipped row against g in fp64 in ascending
+// output order -- the reference's own order, so an int32 payload is the
+// oracle's -- and the item's units are summed over its lanes before one pair of
+// atomics commits the item.  A wave takes `ib` samples and a run of tables, `it`
+// tables a step (ib * it items of `nob` units), with g's block of every lane in
+// registers as fp64 for the whole run.
+//
+// Rows are read coalesced, 8 lanes a 128-byte block, into registers while the
+// step before is computed, and reach the owning lanes through the wave's 16 KiB
+// of LDS (slots swizzled so that neither side meets a bank twice).  What bounds
+// it is the gather where rows are many: the samples of a run of tables share an
+// XCD's L2 (block order) and a step spans few tables, so a selected row crosses
+// HBM once (B = 512, T = 1024, E = 256, O = 256: 298 MB fetched for tables of
+// 268 MB).  With the rows in L2 the two wavefronts a SIMD (228 registers) leave
+// a step's latencies half exposed: 90 us for those 524 k items.  Measured
+// against one wavefront walking all tables of a sample (fp32) and one thread a
+// unit (int32):
+//   fp32   B = 1,   T = 8192, E = 64,  O = 256:   2000 -> 14 us
+//          B = 16,  T = 4096, E = 256, O = 256:   1201 -> 33 us
+//          B = 128, T = 2048, E = 256, O = 1024:   800 -> 295 us (distinct rows: 1.4 GB)
+//   int32  B = 512, T = 1024, E = 256, O = 256:   2975 -> 113 us
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, kWave);
-    return v;
+constexpr int kRowBlock = 32;                       // outputs of a unit
+constexpr int kRowPieces = kRowBlock / 4;           // its 16-byte pieces
+constexpr uint32_t kRowSkip = 0x80000000u;          // an offset past every buffer: loads give 0
+
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int VEC, int SPW, int U>
-__global__ __launch_bounds__(kBlock) void k_propagate_fc_slices(
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+template <bool INT_MODE, bool SCATTER, bool ODD>
+__global__ __launch_bounds__(kWave) void k_propagate_rows(
     const float *__restrict__ w, const float *__restrict__ g, const int32_t *__restrict__ idx,
     const float *__restrict__ md, const int32_t *__restrict__ mi, const int2 *__restrict__ anchors,
-    float *__restrict__ x_grad, uint32_t batch, uint32_t n_inputs, uint32_t n_outputs,
-    uint32_t n_detectors, uint32_t n_anchors, uint32_t n_entries, uint32_t n_slices) {
-    static_assert(U * SPW <= kWave, "one committing lane per (sample, table)");
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = uniform(threadIdx.x / kWave);
-    const uint32_t slice = blockIdx.x % n_slices;
-    const uint32_t b0 = ((blockIdx.x / n_slices) * kWPB + wave) * SPW;
-    if (b0 >= batch) return;
-    const uint32_t c = (slice * kWave + lane) * VEC;
-    const bool active = c < n_outputs;
-    const uint32_t cc = active ? c : 0u;
-    const uint32_t emask = n_entries - 1;
-
-    uint32_t bs[SPW];
-    double gd[SPW][VEC];
-#pragma unroll
-    for (int s = 0; s < SPW; s++) {
-        bs[s] = (b0 + s < batch) ? b0 + s : b0;
-        float gv[VEC];
-        RowLoad<float, VEC>::load(g + (size_t)bs[s] * n_outputs + cc, gv);
-#pragma unroll
-        for (int v = 0; v < VEC; v++) gd[s][v] = active ? (double)gv[v] : 0.0;
+    float *__restrict__ x_grad, uint32_t *__restrict__ du_out, uint32_t batch, uint32_t n_inputs,
+    uint32_t n_outputs, uint32_t n_detectors, uint32_t n_anchors, uint32_t n_entries, uint32_t run, uint32_t n_runs,
+    uint32_t n_obc, uint32_t nob, uint32_t ib, uint32_t it, bool cut_units, double int_rescaler) {
+    __shared__ __attribute__((aligned(16))) u32x4 rows[2][kWave * kRowPieces];
+    const uint32_t lane = threadIdx.x;
+    // all samples of a run of tables on one XCD (workgroup i runs on XCD i % 8)
+    const uint32_t per_run = (batch + ib - 1) / ib * n_obc;
+    uint32_t r, rest;
+    if (n_runs >= 8) {
+        const uint32_t local = blockIdx.x / 8u;
+        r = (local / per_run) * 8u + blockIdx.x % 8u;
+        rest = local % per_run;
+    } else {
+        r = blockIdx.x % n_runs;
+        rest = blockIdx.x / n_runs;
     }
-    // the committing lane j = u*SPW + s handles (sample b0+s, table t+u)
-    const uint32_t my_s = lane % SPW;
-    const uint32_t my_u = lane / SPW;
-    const bool my_live = lane < (uint32_t)(U * SPW) && b0 + my_s < batch;
-    const uint32_t my_b = b0 + (my_live ? my_s : 0u);
+    if (r >= n_runs) return;
+    const uint32_t obc = rest % n_obc;
+    const uint32_t b0 = rest / n_obc * ib;
+    const uint32_t t0 = r * run, t1 = min(t0 + run, n_detectors);
+    // item i is sample b0 + i % ib of the step's table i / ib
+    const uint32_t item = lane / nob, ol = lane % nob;
+    const uint32_t bi = item % ib, ti = item / ib;
+    const uint32_t b = b0 + bi;
+    const uint32_t c0 = (obc * nob + ol) * kRowBlock;
+    const bool unit = ti < it && b < batch && c0 < n_outputs;
+    const uint32_t row_bytes = n_outputs * 4u;
 
-    for (uint32_t t = 0; t < n_detectors; t += U) {
-        float mv[U][SPW][VEC], av[U][SPW][VEC];
+    // lane l moves piece l % 8 of unit 8 i + l / 8; pieces of a row's last block
+    // that lie past the row (they belong to the next one) are skipped by an
+    // offset past the buffer: no branch, so that all loads of a step are in flight
+    const uint32_t piece = lane & 7;
+    uint32_t col[kRowPieces], past[kRowPieces];  // first output of the lane's piece i
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const uint32_t tt = min(t + u, n_detectors - 1);
-            const float *wt = w + (size_t)tt * n_entries * n_outputs + cc;
+    for (int i = 0; i < kRowPieces; i++) {
+        col[i] = (obc * nob + (8u * i + (lane >> 3)) % nob) * kRowBlock + piece * 4u;
+        past[i] = col[i] < n_outputs ? 0u : kRowSkip;
+    }
+    // ODD (n_outputs % 4 != 0): the piece that crosses the row's end holds
+    // values of the next row
+    auto clip = [&](u32x4 v, int i) {
+        if (ODD) {
 #pragma unroll
-            for (int s = 0; s < SPW; s++) {
-                const size_t bt = (size_t)bs[s] * n_detectors + tt;
-                const int32_t m = mi[bt];
-                const uint32_t r = (uint32_t)idx[bt] & emask;
-                const uint32_t ra = (m >= 0 && (uint32_t)m < n_anchors) ? (r ^ (1u << m)) : r;
-                RowLoad<float, VEC>::load(wt + (size_t)r * n_outputs, mv[u][s]);
-                RowLoad<float, VEC>::load(wt + (size_t)ra * n_outputs, av[u][s]);
+            for (int q = 1; q < 4; q++) v[q] = col[i] + q < n_outputs ? v[q] : 0u;
+        }
+        return v;
+    };
+    auto slot_in = [&](int i) {
+        const uint32_t u = 8u * i + (lane >> 3);
+        return u * kRowPieces + (piece ^ ((u >> 1) & 7));
+    };
+    auto slot_out = [&](int k) { return lane * kRowPieces + ((uint32_t)k ^ ((lane >> 1) & 7)); };
+
+    // g's block of this lane; outputs past the row count as 0
+    double gd[kRowBlock];
+    {
+        const float *gb = g + (size_t)b0 * n_outputs;
+        const uint32_t nb = min(ib, batch - b0);
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)gb, (short)0, (int)(nb * row_bytes), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < kRowPieces; i++) {
+            const uint32_t bu = (8u * i + (lane >> 3)) / nob % ib;
+            rows[0][slot_in(i)] = clip(
+                __builtin_amdgcn_raw_buffer_load_b128(rsrc, (bu * row_bytes + col[i] * 4u) | past[i], 0, 0), i);
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < kRowPieces; k++) {
+            const u32x4 v = rows[0][slot_out(k)];
+#pragma unroll
+            for (int q = 0; q < 4; q++) gd[4 * k + q] = (double)__uint_as_float(v[q]);
+        }
+        wave_lds_fence();
+    }
+
+    // an item's lookup, kept by all of its unit lanes
+    struct Key {
+        int32_t row, flip;
+        float margin;
+    };
+    auto load_key = [&](uint32_t tb) {
+        const uint32_t t = tb + ti;
+        Key k{0, -1, 0.0f};
+        if (unit && t < t1) {
+            const size_t bt = (size_t)b * n_detectors + t;
+            k.row = idx[bt];
+            k.flip = mi[bt];
+            k.margin = md[bt];
+        }
+        return k;
+    };
+    u32x4 stage[2][kRowPieces];
+    auto load_rows = [&](uint32_t tb, const Key &k) {
+        const float *wb = w + (size_t)tb * n_entries * n_outputs;
+        const uint64_t left = (uint64_t)(n_detectors - tb) * n_entries * row_bytes;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)wb, (short)0, (int)min(left, (uint64_t)0x7fffffffu), 0x00020000);
+        const bool used = k.flip >= 0 && (uint32_t)k.flip < n_anchors;
+        const uint32_t rm = (uint32_t)k.row & (n_entries - 1);
+        const uint32_t first = ti * n_entries * row_bytes + c0 * 4u;
+        const uint32_t om = used ? first + rm * row_bytes : kRowSkip;
+        const uint32_t oa = used ? first + (rm ^ (1u << k.flip)) * row_bytes : kRowSkip;
+#pragma unroll
+        for (int i = 0; i < kRowPieces; i++) {
+            const int u = 8 * i + (int)(lane >> 3);
+            const uint32_t vm = (uint32_t)__shfl((int)om, u, kWave);
+            const uint32_t va = (uint32_t)__shfl((int)oa, u, kWave);
+            stage[0][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (vm + piece * 16u) | past[i], 0, 0);
+            stage[1][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (va + piece * 16u) | past[i], 0, 0);
+        }
+    };
+    auto store_rows = [&]() {
+#pragma unroll
+        for (int i = 0; i < kRowPieces; i++) {
+            rows[0][slot_in(i)] = clip(stage[0][i], i);
+            rows[1][slot_in(i)] = clip(stage[1][i], i);
+        }
+    };
+
+    Key key = load_key(t0);
+    load_rows(t0, key);
+    Key next = load_key(t0 + it);
+    for (uint32_t tb = t0; tb < t1; tb += it) {
+        store_rows();
+        wave_lds_fence();
+        const Key cur = key;
+        key = next;
+        if (tb + it < t1) {
+            load_rows(tb + it, key);
+            next = load_key(tb + 2 * it);
+        }
+        double ms = 0.0, as = 0.0;
+#pragma unroll
+        for (int h = 0; h < kRowPieces; h += 4) {
+            u32x4 m[4], a[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                m[k] = rows[0][slot_out(h + k)];
+                a[k] = rows[1][slot_out(h + k)];
+            }
+            __builtin_amdgcn_sched_barrier(0);  // all eight LDS reads in flight
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    ms += (double)__uint_as_float(m[k][q]) * gd[4 * (h + k) + q];
+                    as += (double)__uint_as_float(a[k][q]) * gd[4 * (h + k) + q];
+                }
+        }
+        wave_lds_fence();
+        const bool used = cur.flip >= 0 && (uint32_t)cur.flip < n_anchors;
+        double du = du_of_margin(cur.margin) * (ms - as);
+        if (cut_units && !(fabs(du) > kEps)) du = 0.0;
+        int32_t pay = 0;
+        if (INT_MODE) pay = (int32_t)(du * kDenom32 * int_rescaler);
+        for (uint32_t d = 1; d < nob; d <<= 1) {
+            if (INT_MODE) {
+                const int32_t o = __shfl_down(pay, d, kWave);
+                if (ol + d < nob) pay = wrap_add(pay, o);
+            } else {
+                const double o = __shfl_down(du, d, kWave);
+                if (ol + d < nob) du += o;
             }
         }
-        double mine = 0.0;
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-#pragma unroll
-            for (int s = 0; s < SPW; s++) {
-                double p = 0.0;
-#pragma unroll
-                for (int v = 0; v < VEC; v++)
-                    p += ((double)mv[u][s][v] - (double)av[u][s][v]) * gd[s][v];
-                p = wave_sum(p);
-                if (lane == (uint32_t)(u * SPW + s)) mine = p;
+        if (SCATTER) {
+            // one word an item; an item outside the run is another wave's
+            if (unit && ol == 0 && tb + ti < t1) {
+                const bool on = used && (INT_MODE || fabs(du) > kEps);
+                du_out[(size_t)b * n_detectors + tb + ti] =
+                    !on ? 0u : INT_MODE ? (uint32_t)pay : __float_as_uint((float)du);
             }
-        }
-        const uint32_t my_t = t + my_u;
-        if (my_live && my_t < n_detectors) {
-            const size_t bt = (size_t)my_b * n_detectors + my_t;
-            const int32_t m = mi[bt];
-            if (m >= 0 && (uint32_t)m < n_anchors) {
-                const double du = du_of_margin(md[bt]) * mine;
-                if (fabs(du) > kEps) {
-                    const int2 a = anchors[(size_t)my_t * n_anchors + m];
-                    if ((uint32_t)a.x < n_inputs && (uint32_t)a.y < n_inputs) {
-                        float *xg = x_grad + (size_t)my_b * n_inputs;
-                        unsafeAtomicAdd(xg + a.x, (float)du);
-                        unsafeAtomicAdd(xg + a.y, (float)(-du));
-                    }
+        } else if (unit && ol == 0 && used && (INT_MODE ? pay != 0 : fabs(du) > kEps)) {
+            const int2 a = anchors[(size_t)(tb + ti) * n_anchors + cur.flip];
+            if ((uint32_t)a.x < n_inputs && (uint32_t)a.y < n_inputs) {
+                float *xg = x_grad + (size_t)b * n_inputs;
+                if (INT_MODE) {
+                    atomicAdd(reinterpret_cast<int32_t *>(xg + a.x), pay);
+                    atomicAdd(reinterpret_cast<int32_t *>(xg + a.y), (int32_t)(0u - (uint32_t)pay));
+                } else {
+                    unsafeAtomicAdd(xg + a.x, (float)du);
+                    unsafeAtomicAdd(xg + a.y, (float)(-du));
                 }
             }
         }
@@ -788,7 +920,6 @@ __global__ __launch_bounds__(kBlock) void k_wgrad_commit_values(
     cv[i] = v;
 }
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <int VEC>
@@ -986,6 +1117,27 @@ bool rowsum_applies(const FcShape &s) {
     return s.n_entries <= 4096 && (uint64_t)s.batch * s.n_outputs * 4 < 0x7fffffffull;
 }
 
+// Most samples of a step of k_propagate_rows: with more, a step's lookups come
+// from as many lines of the [B][T] index arrays.
+constexpr uint32_t kRowSamples = 8;
+
+// Past 2^14 items the pushes go through du and the LDS scatter: global fp32 and
+// int32 atomics run at about 5 G/s here (B = 512, T = 1024, O = 256, int32:
+// 203 us with a pair of atomics an item), and a small call saves the launch.
+bool propagate_rows_scatters(const FcShape &s) {
+    return input_grad_scatter_applies(s) && (uint64_t)s.batch * s.n_detectors > (1u << 14);
+}
+
+// k_propagate_rows reads a step's tables with 31-bit byte offsets, and forms
+// int32 payloads per 32 outputs.  A few thousand items of a block or less are one
+// wave's work of k_propagate_fc_exact on every CU, without the staging (B = 64,
+// T = 256, O = 10: 7.9 against 8.8 us).
+bool propagate_rows_applies(const FcShape &s, bool int_mode) {
+    if (s.n_outputs <= (uint32_t)kRowBlock && (uint64_t)s.batch * s.n_detectors <= (1u << 14)) return false;
+    if (int_mode && s.ogs != (uint32_t)kRowBlock) return false;
+    return (uint64_t)kWave * s.n_entries * std::max<uint32_t>(s.n_outputs, kRowBlock) * 4 < 0x7fffffffull;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -1066,52 +1218,63 @@ hipError_t launch_fill_fc_i8(const FcShape &s, const int8_t *q8, const float *sc
 #undef SPIKY_FILL_I8
 }
 
+// scratch: du [B][T] u32 for the scattered input gradient, else none
 hipError_t launch_propagate_fc(const FcShape &s, const float *w, const float *g,
                                const int32_t *idx, const float *min_deltas,
                                const int32_t *min_idx, const int32_t *anchors, float *x_grad,
-                               bool int_mode, double int_rescaler, hipStream_t st) {
+                               bool int_mode, double int_rescaler, Scratch &scratch, hipStream_t st) {
+    const bool rows = propagate_rows_applies(s, int_mode);
+    const bool scatter = rows && propagate_rows_scatters(s);
+    ScratchLayout lay(scratch);
+    uint32_t *du = scatter ? lay.take<uint32_t>((size_t)s.batch * s.n_detectors * 4) : nullptr;
+    hipError_t e;
+    if (lay.stop(&e, "propagate_through_detectors_fc")) return e;
     const int2 *ap = reinterpret_cast<const int2 *>(anchors);
-    if (!int_mode && s.n_outputs >= 256) {
-        const uint32_t vec = pick_vec(s.n_outputs);
-        const uint32_t n_slices = (s.n_outputs + kWave * vec - 1) / (kWave * vec);
-        const uint32_t spw = s.batch >= 512 ? 4 : 1;
-        const uint32_t b_groups = (s.batch + kWPB * spw - 1) / (kWPB * spw);
-        const uint64_t grid = (uint64_t)n_slices * b_groups;
+    if (rows) {
+        const uint32_t blocks = (s.n_outputs + kRowBlock - 1) / kRowBlock;
+        const uint32_t n_obc = (blocks + kWave - 1) / kWave;
+        const uint32_t nob = (blocks + n_obc - 1) / n_obc;
+        const uint32_t items = kWave / nob;
+        const uint32_t ib = std::min<uint32_t>({items, s.batch, kRowSamples}), it = items / ib;
+        // steps a wave: one until ~6144 waves (three rounds of 8 a CU) are in the grid
+        const uint64_t groups = (uint64_t)((s.batch + ib - 1) / ib) * n_obc;
+        const uint64_t steps = (s.n_detectors + it - 1) / it * groups;
+        const uint64_t per_wave = std::min<uint64_t>(32, steps / 6144);
+        const uint32_t run = it * (uint32_t)std::max<uint64_t>(1, per_wave);
+        const uint32_t n_runs = (s.n_detectors + run - 1) / run;
+        const uint64_t grid = (uint64_t)(n_runs >= 8 ? (n_runs + 7) / 8 * 8 : n_runs) * groups;
         if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
-#define SPIKY_PROP(V, SPW, U)                                                                     \
-    hipLaunchKernelGGL((k_propagate_fc_slices<V, SPW, U>), dim3((uint32_t)grid), dim3(kBlock), 0, \
-                       st, w, g, idx, min_deltas, min_idx, ap, x_grad, s.batch, s.n_inputs,       \
-                       s.n_outputs, s.n_detectors, s.n_anchors, s.n_entries, n_slices)
-        if (spw == 4) {
-            switch (vec) {
-                case 4: SPIKY_PROP(4, 4, 4); break;
-                case 2: SPIKY_PROP(2, 4, 4); break;
-                default: SPIKY_PROP(1, 4, 4); break;
-            }
+#define SPIKY_PR(IM, SC, ODD)                                                                      \
+    hipLaunchKernelGGL((k_propagate_rows<IM, SC, ODD>), dim3((uint32_t)grid), dim3(kWave), 0, st, w, \
+                       g, idx, min_deltas, min_idx, ap, x_grad, du, s.batch, s.n_inputs, s.n_outputs, \
+                       s.n_detectors, s.n_anchors, s.n_entries, run, n_runs, n_obc, nob, ib, it,    \
+                       s.ogs == (uint32_t)kRowBlock, int_rescaler)
+#define SPIKY_PR_O(IM, SC)                                                                         \
+    if (s.n_outputs % 4 != 0) SPIKY_PR(IM, SC, true); else SPIKY_PR(IM, SC, false)
+        if (scatter) {
+            if (int_mode) { SPIKY_PR_O(true, true); } else { SPIKY_PR_O(false, true); }
         } else {
-            switch (vec) {
-                case 4: SPIKY_PROP(4, 1, 8); break;
-                case 2: SPIKY_PROP(2, 1, 8); break;
-                default: SPIKY_PROP(1, 1, 8); break;
-            }
+            if (int_mode) { SPIKY_PR_O(true, false); } else { SPIKY_PR_O(false, false); }
         }
-#undef SPIKY_PROP
-        return hipGetLastError();
+#undef SPIKY_PR_O
+#undef SPIKY_PR
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        if (scatter) return launch_input_grad_scatter(s, du, min_idx, anchors, x_grad, int_mode, int_rescaler, st);
+    } else {
+        const uint32_t n_ob = (s.n_outputs + s.ogs - 1) / s.ogs;
+        const uint64_t n_items = (uint64_t)s.batch * s.n_detectors * n_ob;
+        if (n_items == 0) return hipSuccess;
+#define SPIKY_PE(IM)                                                                               \
+    hipLaunchKernelGGL(k_propagate_fc_exact<IM>, dim3(blocks_for(n_items)), dim3(kBlock), 0, st, w, \
+                       g, idx, min_deltas, min_idx, ap, x_grad, s.n_inputs, s.n_outputs,            \
+                       s.n_detectors, s.n_anchors, s.n_entries, s.ogs, n_ob, n_items, int_rescaler)
+        if (int_mode) SPIKY_PE(true); else SPIKY_PE(false);
+#undef SPIKY_PE
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
     }
-    const uint32_t n_ob = (s.n_outputs + s.ogs - 1) / s.ogs;
-    const uint64_t n_items = (uint64_t)s.batch * s.n_detectors * n_ob;
-    if (n_items == 0) return hipSuccess;
-    if (int_mode)
-        hipLaunchKernelGGL(k_propagate_fc_exact<true>, dim3(blocks_for(n_items)), dim3(kBlock), 0,
-                           st, w, g, idx, min_deltas, min_idx, ap, x_grad, s.n_inputs,
-                           s.n_outputs, s.n_detectors, s.n_anchors, s.n_entries, s.ogs, n_ob,
-                           n_items, int_rescaler);
-    else
-        hipLaunchKernelGGL(k_propagate_fc_exact<false>, dim3(blocks_for(n_items)), dim3(kBlock),
-                           0, st, w, g, idx, min_deltas, min_idx, ap, x_grad, s.n_inputs,
-                           s.n_outputs, s.n_detectors, s.n_anchors, s.n_entries, s.ogs, n_ob,
-                           n_items, int_rescaler);
-    return hipGetLastError();
+    return int_mode ? launch_convert_i2f(x_grad, (uint64_t)s.batch * s.n_inputs, int_rescaler, st) : hipSuccess;
 }
 
 // scratch (bucketed path): bucket offsets [T][E+1] | sorted samples [T][B] |

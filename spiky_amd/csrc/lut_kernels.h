@@ -113,11 +113,22 @@ hipError_t launch_fill_fc_i8(const FcShape &s, const int8_t *q8, const float *sc
                              const int32_t *idx, float *out, bool int_mode, double int_rescaler,
                              hipStream_t st);
 
-// Min-margin input gradient.
+// Min-margin input gradient; int_mode sums int32 payloads into x_grad's words
+// and leaves it converted to fp32.  Scratch: du [B][T] where the input gradient
+// is scattered from it.
 hipError_t launch_propagate_fc(const FcShape &s, const float *w, const float *g,
                                const int32_t *idx, const float *min_deltas,
                                const int32_t *min_idx, const int32_t *anchors, float *x_grad,
-                               bool int_mode, double int_rescaler, hipStream_t st);
+                               bool int_mode, double int_rescaler, Scratch &scratch, hipStream_t st);
+
+// x_grad[b][a1] += du, x_grad[b][a2] -= du at the min-margin pair of every
+// (sample, table); du [B][T] holds fp32 terms, or int32 payloads in int_mode
+// (x_grad is then converted to fp32).  0 marks no term.  Applies while a
+// sample's input row fits the LDS sums.
+bool input_grad_scatter_applies(const FcShape &s);
+hipError_t launch_input_grad_scatter(const FcShape &s, const uint32_t *du, const int32_t *min_idx,
+                                     const int32_t *anchors, float *x_grad, bool int_mode,
+                                     double int_rescaler, hipStream_t st);
 
 // Table-row gradient: target[row, o] += lr * g[b, o] for every sample b hitting row.
 // The bucketed path lays out its buckets and commit values in scratch (none for

@@ -1008,23 +1008,28 @@ __global__ __launch_bounds__(256) void k_propagate_reduce(const float *__restric
     }
 }
 
-// x_grad[b][a1] += du, x_grad[b][a2] -= du for every table with |du| > EPS
+// x_grad[b][a1] += du, x_grad[b][a2] -= du for every table whose du is not 0
 // (propagate_through_detector, proto:821-867).  One workgroup per group of
-// samples; their input-gradient rows are accumulated in LDS and added to HBM
-// once.
+// samples; their input-gradient rows are accumulated in LDS (LDS_BYTES) and
+// added to HBM once.  int32 summation: du holds the payloads, the sums wrap,
+// and the row is converted to fp32 as it is written.
 constexpr int kScatterThreads = 1024;
 constexpr int kScatterLds = 128 * 1024;
+constexpr int kScatterLdsSmall = 32 * 1024;  // lets two workgroups share a CU
 
+template <bool INT_MODE, int LDS_BYTES>
 __global__ __launch_bounds__(kScatterThreads) void k_propagate_scatter(
-    const float *__restrict__ du_in, const int32_t *__restrict__ mi,
+    const uint32_t *__restrict__ du_in, const int32_t *__restrict__ mi,
     const int2 *__restrict__ anchors, float *__restrict__ x_grad, uint32_t batch,
-    uint32_t n_inputs, uint32_t n_detectors, uint32_t n_anchors, uint32_t samples_per_group) {
+    uint32_t n_inputs, uint32_t n_detectors, uint32_t n_anchors, uint32_t samples_per_group,
+    double int_rescaler) {
     // fp64 sums: on gfx950 ds_add_f64 sustains ~20x the lanes a clock of ds_add_f32
-    __shared__ double xg[kScatterLds / 8];
+    using Sum = typename std::conditional<INT_MODE, uint32_t, double>::type;
+    __shared__ Sum xg[LDS_BYTES / 8];
     const uint32_t b0 = blockIdx.x * samples_per_group;
     const uint32_t nb = min(samples_per_group, batch - b0);
     const uint32_t n_el = nb * n_inputs;
-    for (uint32_t i = threadIdx.x; i < n_el; i += kScatterThreads) xg[i] = 0.0;
+    for (uint32_t i = threadIdx.x; i < n_el; i += kScatterThreads) xg[i] = (Sum)0;
     __syncthreads();
     const uint32_t n_pairs = nb * n_detectors;
     const size_t base = (size_t)b0 * n_detectors;
@@ -1032,32 +1037,49 @@ __global__ __launch_bounds__(kScatterThreads) void k_propagate_scatter(
     // loads, then their anchor loads, each batch in flight together
     constexpr int kU = 8;
     for (uint32_t p0 = threadIdx.x; p0 < n_pairs; p0 += kU * kScatterThreads) {
-        float du[kU];
+        uint32_t du[kU];
         int32_t m[kU];
 #pragma unroll
         for (int u = 0; u < kU; u++) {
             const uint32_t p = p0 + u * kScatterThreads;
-            du[u] = p < n_pairs ? du_in[base + p] : 0.0f;
+            du[u] = p < n_pairs ? du_in[base + p] : 0u;
             m[u] = p < n_pairs ? mi[base + p] : -1;
         }
         int2 a[kU];
 #pragma unroll
         for (int u = 0; u < kU; u++) {
             const uint32_t t = (p0 + u * kScatterThreads) % n_detectors;
-            const bool on = du[u] != 0.0f && m[u] >= 0 && (uint32_t)m[u] < n_anchors;
+            const bool some = INT_MODE ? du[u] != 0u : __uint_as_float(du[u]) != 0.0f;
+            const bool on = some && m[u] >= 0 && (uint32_t)m[u] < n_anchors;
             a[u] = on ? anchors[(size_t)t * n_anchors + m[u]] : make_int2(-1, -1);
         }
 #pragma unroll
         for (int u = 0; u < kU; u++) {
             if ((uint32_t)a[u].x >= n_inputs || (uint32_t)a[u].y >= n_inputs) continue;
             const uint32_t bl = (p0 + u * kScatterThreads) / n_detectors;
-            atomicAdd(&xg[bl * n_inputs + a[u].x], (double)du[u]);
-            atomicAdd(&xg[bl * n_inputs + a[u].y], -(double)du[u]);
+            Sum up, down;
+            if constexpr (INT_MODE) {
+                up = du[u];
+                down = 0u - du[u];
+            } else {
+                up = (double)__uint_as_float(du[u]);
+                down = -up;
+            }
+            atomicAdd(&xg[bl * n_inputs + a[u].x], up);
+            atomicAdd(&xg[bl * n_inputs + a[u].y], down);
         }
     }
     __syncthreads();
     float *dst = x_grad + (size_t)b0 * n_inputs;
-    for (uint32_t i = threadIdx.x; i < n_el; i += kScatterThreads) dst[i] += (float)xg[i];
+    for (uint32_t i = threadIdx.x; i < n_el; i += kScatterThreads) {
+        if constexpr (INT_MODE) {
+            // convert_integers_to_floats_logic, proto:200-213
+            const int32_t v = (int32_t)(__float_as_uint(dst[i]) + xg[i]);
+            dst[i] = (float)(((double)v * kDenom32Reciproc) / int_rescaler);
+        } else {
+            dst[i] += (float)xg[i];
+        }
+    }
 }
 
 // keys_t[t][b] = idx[b][t] & emask (u8), through a 64x64 LDS tile: the rows the
@@ -1331,16 +1353,13 @@ hipError_t launch_block_commit(const uint32_t *part, float *out, uint64_t n, uin
 bool tm_propagate_applies(const FcShape &s) {
     const uint64_t n_slices = (s.n_outputs + kTmCols - 1) / kTmCols;
     return s.batch >= 256 && s.n_entries <= (uint32_t)kTmMaxEntries && s.n_outputs % 4 == 0 &&
-           s.n_outputs >= 64 && s.n_inputs * 8 <= (uint32_t)kScatterLds &&
+           s.n_outputs >= 64 && input_grad_scatter_applies(s) &&
            n_slices * s.batch * s.n_detectors * 4 <= (4ull << 30);
 }
 
 static hipError_t launch_propagate_finish(const FcShape &s, float *dpart, uint32_t n_slices,
                                           const float *min_deltas, const int32_t *min_idx,
                                           const int32_t *anchors, float *x_grad, hipStream_t st);
-static hipError_t launch_propagate_scatter(const FcShape &s, const float *du, const int32_t *min_idx,
-                                           const int32_t *anchors, float *x_grad, hipStream_t st);
-
 // the 64-column propagate: whole 256-row fp32 tables, 64-column slices
 static bool tm_propagate_wide(const FcShape &s) {
     // k_propagate_units reads g with 32-bit byte offsets, up to a whole chunk
@@ -1429,7 +1448,8 @@ hipError_t launch_propagate_tm(const FcShape &s, const float *w, const float *g,
 #undef SPIKY_PU
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        return launch_propagate_scatter(s, du, min_idx, anchors, x_grad, st);
+        return launch_input_grad_scatter(s, reinterpret_cast<const uint32_t *>(du), min_idx, anchors, x_grad,
+                                         false, 1.0, st);
     }
     // the LDS-DMA ring needs whole 256-row tables
     const bool dma = s.n_entries == (uint32_t)kTmMaxEntries;
@@ -1470,17 +1490,30 @@ static hipError_t launch_propagate_finish(const FcShape &s, float *dpart, uint32
                        s.n_anchors, n_slices, s.ogs == (uint32_t)kTmCols);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_propagate_scatter(s, du, min_idx, anchors, x_grad, st);
+    return launch_input_grad_scatter(s, reinterpret_cast<const uint32_t *>(du), min_idx, anchors, x_grad,
+                                     false, 1.0, st);
 }
 
-// x_grad from du [B][T]
-static hipError_t launch_propagate_scatter(const FcShape &s, const float *du, const int32_t *min_idx,
-                                           const int32_t *anchors, float *x_grad, hipStream_t st) {
-    const uint32_t spg = std::max<uint32_t>(1, std::min<uint32_t>(16, kScatterLds / 8 / s.n_inputs));
+bool input_grad_scatter_applies(const FcShape &s) { return (uint64_t)s.n_inputs * 8 <= (uint64_t)kScatterLds; }
+
+hipError_t launch_input_grad_scatter(const FcShape &s, const uint32_t *du, const int32_t *min_idx,
+                                     const int32_t *anchors, float *x_grad, bool int_mode,
+                                     double int_rescaler, hipStream_t st) {
+    // samples a workgroup: as few as leaves a workgroup a CU, at most 16 or what LDS holds
+    const uint32_t spg = std::max<uint32_t>(
+        1, std::min<uint32_t>({16u, (uint32_t)kScatterLds / 8 / s.n_inputs, s.batch / 256}));
     const uint32_t groups = (s.batch + spg - 1) / spg;
-    hipLaunchKernelGGL(k_propagate_scatter, dim3(groups), dim3(kScatterThreads), 0, st, du,
-                       min_idx, reinterpret_cast<const int2 *>(anchors), x_grad, s.batch,
-                       s.n_inputs, s.n_detectors, s.n_anchors, spg);
+    const bool small = (uint64_t)spg * s.n_inputs * 8 <= (uint64_t)kScatterLdsSmall;
+#define SPIKY_PS(IM, LDS)                                                                          \
+    hipLaunchKernelGGL((k_propagate_scatter<IM, LDS>), dim3(groups), dim3(kScatterThreads), 0, st,  \
+                       du, min_idx, reinterpret_cast<const int2 *>(anchors), x_grad, s.batch,       \
+                       s.n_inputs, s.n_detectors, s.n_anchors, spg, int_rescaler)
+    if (int_mode) {
+        if (small) SPIKY_PS(true, kScatterLdsSmall); else SPIKY_PS(true, kScatterLds);
+    } else {
+        if (small) SPIKY_PS(false, kScatterLdsSmall); else SPIKY_PS(false, kScatterLds);
+    }
+#undef SPIKY_PS
     return hipGetLastError();
 }
 

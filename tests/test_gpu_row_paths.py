@@ -1,0 +1,54 @@
+"""GPU parity of the gathered-row kernels of the fully connected path (small
+batches, odd output counts, many rows a table) against the CPU oracle, at the
+edges of their units: 32-output blocks, 16-byte pieces, samples and tables a
+step, and rows that end inside a piece."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_fc import make_dm, make_inputs, run_fc, xg_close
+
+pytestmark = pytest.mark.gpu
+
+
+# B, T, Nc, O: a lone sample; one output; a block and one output more or less;
+# sample groups and tables that are not whole; more blocks than lanes (two
+# chunks); 512 rows a table; past the direct pushes (B * T > 2^14)
+@pytest.mark.parametrize("int_rescaler", [None, 0.5])
+@pytest.mark.parametrize("B,T,Nc,O", [(1, 70, 4, 33), (1, 600, 3, 2), (9, 37, 5, 31), (7, 40, 4, 301),
+                                      (3, 9, 2, 2049), (2, 5, 2, 4100), (17, 33, 9, 96),
+                                      (40, 430, 4, 63), (130, 130, 3, 5)])
+def test_propagate_rows(oracle, cuda_device, B, T, Nc, O, int_rescaler):
+    run_fc(oracle, B, 48, T, Nc, O, seed=B + O, int_rescaler=int_rescaler)
+
+
+@pytest.mark.parametrize("O", [10, 33, 301])
+def test_rows_not_looked_up_are_not_read(oracle, cuda_device, O):
+    """Rows that no sample selects hold NaN: a row whose last piece crosses into
+    one gives the oracle's gradients, which never touch it."""
+    B, I, T, Nc = 6, 40, 25, 6
+    E = 1 << Nc
+    x, anchors, W, go = make_inputs(5, B, I, T, Nc, O)
+    ridx, rmd, rmi = oracle.check_detectors(x.numpy(), anchors.numpy(), B, I, T, Nc)
+    used = np.zeros((T, E), bool)
+    rows = ridx.reshape(B, T)
+    flip = rows ^ (1 << rmi.reshape(B, T))
+    for t in range(T):
+        used[t, rows[:, t]] = used[t, flip[:, t]] = True
+    W = W.view(T, E, O)
+    W[torch.from_numpy(~used)] = float("nan")
+    W = W.reshape(-1).contiguous()
+    dm = make_dm(I, O, T, Nc)
+    dev = torch.device("cuda:0")
+    xd, ad, Wd, gd = (v.to(dev) for v in (x, anchors, W, go))
+    out, xg = torch.zeros(B * O, device=dev), torch.zeros(B * I, device=dev)
+    idx = torch.empty(B * T, dtype=torch.int32, device=dev)
+    md, mi = torch.empty(B * T, device=dev), torch.empty(B * T, dtype=torch.int32, device=dev)
+    wg = torch.empty(T * E * O, device=dev)
+    print(f"[rows] O={O}", flush=True)
+    dm.forward_step(Wd, B, xd, ad, out, idx, 0.0, None, md, mi)
+    dm.backward_backprop(Wd, B, gd, ad, idx, md, mi, xg, -1.0, wg, None, overwrite_weights_gradients=True)
+    rxg = oracle.propagate_fc(W.numpy(), go.numpy(), ridx, rmd, rmi, anchors.numpy(), B, I, O, T, Nc, E)
+    assert np.array_equal(out.cpu().numpy(), oracle.fill_outputs_fc(W.numpy(), ridx, B, O, T, E))
+    assert np.all(np.isfinite(rxg))
+    xg_close(xg.cpu().numpy(), rxg, B, I, T, (O + 31) // 32)
