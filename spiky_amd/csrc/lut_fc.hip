@@ -10,13 +10,11 @@
 // Kernels and their schedules:
 //   k_check_detectors   one thread per table over the x rows of a few samples
 //                       staged in LDS (one thread per (b, t) for very wide x).
-//   k_fill_fc           one wavefront per (sample, column slice of 64*VEC);
-//                       slices are mapped to XCDs (workgroup id mod 8) so each
-//                       XCD's L2 serves one column slice of every table to all
-//                       samples; each lane owns VEC columns and walks the tables
-//                       in ascending order with fp64 partials per block of `dgs`
-//                       tables and an fp32 (or int32) running sum -- the exact
-//                       commit order of the reference CPU path, so the output is
+//   k_fill_blocks       one workgroup per (sample, column slice): a thread sums
+//                       a block of `dgs` tables of a few columns in fp64, and
+//                       the blocks' fp32 (or int32) commit values are added in
+//                       ascending order through LDS -- the exact commit order
+//                       of the reference CPU path, so the output is
 //                       bit-identical to it.
 //   k_propagate_rows    one wavefront per (few samples, run of tables); a lane
 //                       owns a 32-output block of a (sample, table) item, fed
@@ -252,148 +250,172 @@ uint32_t pick_vec(uint32_t n_outputs) {
     return 1;
 }
 
-// Forward gather-sum.  Wavefront = SPW samples x one column slice; each lane
-// owns VEC columns of every sample and walks the tables in ascending order,
-// with an fp64 partial per block of `dgs` tables and an fp32 (or int32) running
-// sum -- the reference CPU path's exact commit order, so the output is
-// bit-identical to it.  U tables x SPW samples of row loads are issued before
-// the ordered adds.  Sample and column indices past the end are clamped to
-// valid memory for the loads and masked at the store.
-template <typename WT, int VEC, int SPW, int U, bool INT_MODE, bool SCALED>
-__global__ __launch_bounds__(kBlock) void k_fill_fc(
-    const WT *__restrict__ w, const float *__restrict__ scales, const int32_t *__restrict__ idx,
-    float *__restrict__ out, uint32_t batch, uint32_t n_outputs, uint32_t n_detectors,
-    uint32_t n_entries, uint32_t dgs, uint32_t n_slices, double int_rescaler) {
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = uniform(threadIdx.x / kWave);
-    const uint32_t slice = blockIdx.x % n_slices;
-    const uint32_t b0 = ((blockIdx.x / n_slices) * kWPB + wave) * SPW;
-    if (b0 >= batch) return;
-    const uint32_t c = (slice * kWave + lane) * VEC;
-    const bool active = c < n_outputs;
-    const uint32_t cc = active ? c : 0u;
-    const uint32_t emask = n_entries - 1;
-    const int32_t *ib[SPW];
-    bool live[SPW];
-#pragma unroll
-    for (int s = 0; s < SPW; s++) {
-        live[s] = b0 + s < batch;
-        ib[s] = idx + (size_t)(live[s] ? b0 + s : b0) * n_detectors;
-    }
+// Forward gather-sum.  A workgroup owns a sample's column slice, a thread VEC
+// columns of one block of dgs tables at a time (16 rows in flight, fp64,
+// ascending tables); the blocks' commit values meet
+// in LDS and are added in ascending block order: the reference CPU path's
+// arithmetic and commit order, so the output is bit-identical to it, and no
+// scratch.  What bounds it is the gather (B = 128, T = 2048, E = 256, O = 1024:
+// 170 us, 1.1 GB of rows at 6.3 TB/s) and, for a lone sample, its few dependent
+// loads.  One wavefront a column slice walking all tables in order, which this
+// replaces, had 16 rows in flight a slice and paid a load latency for every 16
+// tables:
+//   fp32  B = 1,    T = 8192, E = 256,  O = 1024:  532 -> 26 us
+//         B = 16,   T = 4096, E = 256,  O = 256:   255 -> 18 us
+//         B = 100,  T = 1000, E = 128,  O = 301:    72 -> 24 us
+//         B = 1024, T = 1024, E = 1024, O = 256:   244 -> 165 us
+//   int8  B = 32,   T = 4096, E = 256,  O = 1024:  399 -> 43 us
+//
+// A quad that would cross the row's end starts at n_outputs - 4 instead: its
+// first columns repeat the quad before it, value for value.
+constexpr int kBlocksThreads = 1024;
+constexpr uint32_t kBlocksLds = 8448;  // most commit values in LDS (33 KiB): 234 blocks of 32 columns + 4
 
-    float run[SPW][VEC];
-    int32_t irun[SPW][VEC];
-#pragma unroll
-    for (int s = 0; s < SPW; s++) {
-#pragma unroll
-        for (int v = 0; v < VEC; v++) {
-            run[s][v] = 0.0f;
-            irun[s][v] = 0;
-            if (active && live[s]) {
-                const float o = out[(size_t)(b0 + s) * n_outputs + c + v];
-                if (INT_MODE)
-                    irun[s][v] = __float_as_int(o);
-                else
-                    run[s][v] = o;
-            }
-        }
-    }
+typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-    for (uint32_t t0 = 0; t0 < n_detectors; t0 += dgs) {
-        const uint32_t t1 = min(t0 + dgs, n_detectors);
-        double acc[SPW][VEC];
+template <typename WT, int VEC>
+__device__ __forceinline__ void load_columns(const WT *p, float *v) {
+    if constexpr (VEC == 4 && sizeof(WT) == 4) {
+        const f32x4u q = *reinterpret_cast<const f32x4u *>(p);
 #pragma unroll
-        for (int s = 0; s < SPW; s++)
-#pragma unroll
-            for (int v = 0; v < VEC; v++) acc[s][v] = 0.0;
-        uint32_t t = t0;
-        for (; t + U <= t1; t += U) {
-            float vals[U][SPW][VEC];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const WT *wt = w + (size_t)(t + u) * n_entries * n_outputs + cc;
-#pragma unroll
-                for (int s = 0; s < SPW; s++) {
-                    const uint32_t r = (uint32_t)ib[s][t + u] & emask;
-                    RowLoad<WT, VEC>::load(wt + (size_t)r * n_outputs, vals[u][s]);
-                }
-                if (SCALED) {
-                    const float sc = scales[t + u];
-#pragma unroll
-                    for (int s = 0; s < SPW; s++)
-#pragma unroll
-                        for (int v = 0; v < VEC; v++) vals[u][s][v] = sc * vals[u][s][v];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int s = 0; s < SPW; s++)
-#pragma unroll
-                    for (int v = 0; v < VEC; v++) acc[s][v] += (double)vals[u][s][v];
-        }
-        for (; t < t1; t++) {
-            const WT *wt = w + (size_t)t * n_entries * n_outputs + cc;
-            float vals[SPW][VEC];
-#pragma unroll
-            for (int s = 0; s < SPW; s++) {
-                const uint32_t r = (uint32_t)ib[s][t] & emask;
-                RowLoad<WT, VEC>::load(wt + (size_t)r * n_outputs, vals[s]);
-            }
-            const float sc = SCALED ? scales[t] : 1.0f;
-#pragma unroll
-            for (int s = 0; s < SPW; s++)
-#pragma unroll
-                for (int v = 0; v < VEC; v++)
-                    acc[s][v] += (double)(SCALED ? sc * vals[s][v] : vals[s][v]);
-        }
-#pragma unroll
-        for (int s = 0; s < SPW; s++)
-#pragma unroll
-            for (int v = 0; v < VEC; v++) {
-                if (INT_MODE)
-                    irun[s][v] = wrap_add(irun[s][v], (int32_t)(acc[s][v] * kDenom32 * int_rescaler));
-                else
-                    run[s][v] += (float)acc[s][v];
-            }
-    }
-    if (!active) return;
-#pragma unroll
-    for (int s = 0; s < SPW; s++) {
-        if (!live[s]) continue;
-        float *ob = out + (size_t)(b0 + s) * n_outputs + c;
-#pragma unroll
-        for (int v = 0; v < VEC; v++) {
-            if (INT_MODE) {
-                // convert_integers_to_floats_logic, proto:200-213
-                const double y = (double)irun[s][v] * kDenom32Reciproc;
-                ob[v] = (float)(y / int_rescaler);
-            } else {
-                ob[v] = run[s][v];
-            }
-        }
+        for (int i = 0; i < 4; i++) v[i] = q[i];
+    } else {
+        RowLoad<WT, VEC>::load(p, v);
     }
 }
 
 template <typename WT, int VEC, bool INT_MODE, bool SCALED>
-hipError_t launch_fill_variant(const FcShape &s, const WT *w, const float *scales,
-                               const int32_t *idx, float *out, double int_rescaler,
-                               hipStream_t st) {
-    const uint32_t n_slices = (s.n_outputs + kWave * VEC - 1) / (kWave * VEC);
-    // several samples per wavefront once the batch is large enough to fill the chip
-    const uint32_t spw = s.batch >= 512 ? 4 : 1;
-    const uint32_t b_groups = (s.batch + kWPB * spw - 1) / (kWPB * spw);
-    const uint64_t grid = (uint64_t)n_slices * b_groups;
-    if (grid == 0) return hipSuccess;
+__global__ __launch_bounds__(kBlocksThreads) void k_fill_blocks(
+    const WT *__restrict__ w, const float *__restrict__ scales, const int32_t *__restrict__ idx,
+    float *__restrict__ out, uint32_t n_outputs, uint32_t n_detectors, uint32_t n_entries,
+    uint32_t dgs, uint32_t nq, uint32_t n_slices, uint32_t n_blocks, uint32_t cap, double int_rescaler) {
+    extern __shared__ uint32_t part[];  // a row of commit values for each block of a chunk
+    constexpr int U = 16;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t slice = blockIdx.x % n_slices;
+    const uint32_t b = blockIdx.x / n_slices;
+    const uint32_t c0 = slice * nq * VEC;
+    const uint32_t nc = min(nq * VEC, n_outputs - c0);
+    const uint32_t q = tid % nq, g = tid / nq, groups = blockDim.x / nq;
+    const uint32_t c = c0 + q * VEC;
+    const bool on = g < groups && c < n_outputs;
+    const uint32_t cs = min(c, n_outputs - VEC);  // n_outputs >= VEC
+    const uint32_t width = nq * VEC + VEC;         // of a block's row in LDS, VEC spare columns first
+    const uint32_t emask = n_entries - 1;
+    const int32_t *ib = idx + (size_t)b * n_detectors;
+    const WT *wc = w + cs;
+    const size_t table = (size_t)n_entries * n_outputs;
+
+    // the lookups of tables t .. t + U - 1 (past the last table: its lookup)
+    auto lookups = [&](uint32_t (&r)[U], uint32_t t) {
+        if (t + U <= n_detectors) {
+#pragma unroll
+            for (int u = 0; u < U; u += 4) {
+                const i32x4u iv = *reinterpret_cast<const i32x4u *>(ib + t + u);
+#pragma unroll
+                for (int i = 0; i < 4; i++) r[u + i] = (uint32_t)iv[i] & emask;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) r[u] = (uint32_t)ib[min(t + u, n_detectors - 1)] & emask;
+        }
+    };
+
+    // the summing threads carry the running output over the chunks of blocks
+    float run = 0.0f;
+    int32_t irun = 0;
+    float *op = out + (size_t)b * n_outputs + c0 + tid;
+    if (tid < nc) {
+        run = *op;
+        irun = __float_as_int(run);
+    }
+    for (uint32_t k0 = 0; k0 < n_blocks; k0 += cap) {
+        const uint32_t nk = min(cap, n_blocks - k0);
+        for (uint32_t k = g; on && k < nk; k += groups) {
+            const uint32_t t0 = (k0 + k) * dgs;
+            const uint32_t t1 = min(t0 + dgs, n_detectors);
+            double acc[VEC];
+#pragma unroll
+            for (int v = 0; v < VEC; v++) acc[v] = 0.0;
+            for (uint32_t t = t0; t < t1; t += U) {
+                uint32_t r[U];
+                lookups(r, t);
+                float vals[U][VEC];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const uint32_t tt = min(t + u, n_detectors - 1);
+                    load_columns<WT, VEC>(wc + tt * table + (size_t)r[u] * n_outputs, vals[u]);
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const float sc = SCALED ? scales[min(t + u, n_detectors - 1)] : 1.0f;
+#pragma unroll
+                    for (int v = 0; v < VEC; v++) {
+                        const float x = SCALED ? sc * vals[u][v] : vals[u][v];
+                        acc[v] += t + u < t1 ? (double)x : 0.0;
+                    }
+                }
+            }
+            uint32_t *row = part + k * width + VEC + cs - c0;
+#pragma unroll
+            for (int v = 0; v < VEC; v++)
+                row[v] = INT_MODE ? (uint32_t)(int32_t)(acc[v] * kDenom32 * int_rescaler)
+                                  : __float_as_uint((float)acc[v]);
+        }
+        __syncthreads();
+        if (tid < nc) {
+            const uint32_t *col = part + VEC + tid;
+            uint32_t k = 0;
+            for (; k + U <= nk; k += U) {
+                uint32_t v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) v[u] = col[(k + u) * width];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    if (INT_MODE)
+                        irun = wrap_add(irun, (int32_t)v[u]);
+                    else
+                        run += __uint_as_float(v[u]);
+                }
+            }
+            for (; k < nk; k++) {
+                if (INT_MODE)
+                    irun = wrap_add(irun, (int32_t)col[k * width]);
+                else
+                    run += __uint_as_float(col[k * width]);
+            }
+        }
+        __syncthreads();
+    }
+    if (tid < nc)
+        // convert_integers_to_floats_logic, proto:200-213
+        *op = INT_MODE ? (float)(((double)irun * kDenom32Reciproc) / int_rescaler) : run;
+}
+
+template <typename WT, int VEC, bool INT_MODE, bool SCALED>
+hipError_t launch_fill_blocks(const FcShape &s, const WT *w, const float *scales, const int32_t *idx,
+                              float *out, double int_rescaler, hipStream_t st) {
+    // slices of up to 64 quads, fewer where the batch alone leaves the 256 CUs
+    // idle, down to 8 (128 bytes of a row; a lone sample's 4): B = 1, O = 1024:
+    // 27 us at 4 quads, 29 at 8, 121 at 64; B = 16: 102 at 16, 188 at 64;
+    // B = 255, O = 1000: 510 at 8, 341 at 64
+    const uint32_t quads = (s.n_outputs + VEC - 1) / VEC;
+    uint32_t n_slices = std::min<uint32_t>((quads + 7) / 8, 256 / s.batch);
+    if ((uint64_t)s.batch * n_slices < 64) n_slices = std::min<uint32_t>((quads + 3) / 4, 256 / s.batch);
+    n_slices = std::max<uint32_t>(n_slices, (quads + 63) / 64);
+    const uint32_t nq = (quads + n_slices - 1) / n_slices;
+    n_slices = (quads + nq - 1) / nq;  // every slice starts inside the row
+    const uint32_t n_blocks = (s.n_detectors + s.dgs - 1) / s.dgs;
+    const uint64_t grid = (uint64_t)n_slices * s.batch;
     if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
-    if (spw == 4)
-        hipLaunchKernelGGL((k_fill_fc<WT, VEC, 4, 8, INT_MODE, SCALED>), dim3((uint32_t)grid),
-                           dim3(kBlock), 0, st, w, scales, idx, out, s.batch, s.n_outputs,
-                           s.n_detectors, s.n_entries, s.dgs, n_slices, int_rescaler);
-    else
-        hipLaunchKernelGGL((k_fill_fc<WT, VEC, 1, 16, INT_MODE, SCALED>), dim3((uint32_t)grid),
-                           dim3(kBlock), 0, st, w, scales, idx, out, s.batch, s.n_outputs,
-                           s.n_detectors, s.n_entries, s.dgs, n_slices, int_rescaler);
+    const uint64_t want = std::max<uint64_t>((uint64_t)nq * n_blocks, nq * VEC);
+    const uint32_t threads = (uint32_t)std::min<uint64_t>(kBlocksThreads, (want + kWave - 1) / kWave * kWave);
+    const uint32_t width = nq * VEC + VEC;
+    const uint32_t cap = std::min<uint32_t>(n_blocks, kBlocksLds / width);  // blocks of a chunk
+    hipLaunchKernelGGL((k_fill_blocks<WT, VEC, INT_MODE, SCALED>), dim3((uint32_t)grid), dim3(threads),
+                       cap * width * 4, st, w, scales, idx, out, s.n_outputs, s.n_detectors, s.n_entries,
+                       s.dgs, nq, n_slices, n_blocks, cap, int_rescaler);
     return hipGetLastError();
 }
 
@@ -1187,35 +1209,26 @@ hipError_t launch_check_detectors(const FcShape &s, const float *x, const int32_
     return hipGetLastError();
 }
 
+template <typename WT, bool INT_MODE, bool SCALED>
+static hipError_t launch_fill_fc(const FcShape &s, const WT *w, const float *scales, const int32_t *idx,
+                                 float *out, double int_rescaler, hipStream_t st) {
+    if ((uint64_t)s.batch * s.n_detectors * s.n_outputs == 0) return hipSuccess;
+    if (s.n_outputs >= 4 && (sizeof(WT) == 4 || s.n_outputs % 4 == 0))
+        return launch_fill_blocks<WT, 4, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st);
+    return launch_fill_blocks<WT, 1, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st);
+}
+
 hipError_t launch_fill_fc_f32(const FcShape &s, const float *w, const int32_t *idx, float *out,
                               bool int_mode, double int_rescaler, hipStream_t st) {
-#define SPIKY_FILL_F32(V)                                                                        \
-    return int_mode ? launch_fill_variant<float, V, true, false>(s, w, nullptr, idx, out,        \
-                                                                 int_rescaler, st)               \
-                    : launch_fill_variant<float, V, false, false>(s, w, nullptr, idx, out,       \
-                                                                  int_rescaler, st)
-    switch (pick_vec(s.n_outputs)) {
-        case 4: SPIKY_FILL_F32(4);
-        case 2: SPIKY_FILL_F32(2);
-        default: SPIKY_FILL_F32(1);
-    }
-#undef SPIKY_FILL_F32
+    return int_mode ? launch_fill_fc<float, true, false>(s, w, nullptr, idx, out, int_rescaler, st)
+                    : launch_fill_fc<float, false, false>(s, w, nullptr, idx, out, int_rescaler, st);
 }
 
 hipError_t launch_fill_fc_i8(const FcShape &s, const int8_t *q8, const float *scales,
                              const int32_t *idx, float *out, bool int_mode, double int_rescaler,
                              hipStream_t st) {
-#define SPIKY_FILL_I8(V)                                                                         \
-    return int_mode ? launch_fill_variant<int8_t, V, true, true>(s, q8, scales, idx, out,        \
-                                                                 int_rescaler, st)               \
-                    : launch_fill_variant<int8_t, V, false, true>(s, q8, scales, idx, out,       \
-                                                                  int_rescaler, st)
-    switch (pick_vec(s.n_outputs)) {
-        case 4: SPIKY_FILL_I8(4);
-        case 2: SPIKY_FILL_I8(2);
-        default: SPIKY_FILL_I8(1);
-    }
-#undef SPIKY_FILL_I8
+    return int_mode ? launch_fill_fc<int8_t, true, true>(s, q8, scales, idx, out, int_rescaler, st)
+                    : launch_fill_fc<int8_t, false, true>(s, q8, scales, idx, out, int_rescaler, st);
 }
 
 // scratch: du [B][T] u32 for the scattered input gradient, else none

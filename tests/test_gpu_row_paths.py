@@ -52,3 +52,38 @@ def test_rows_not_looked_up_are_not_read(oracle, cuda_device, O):
     assert np.array_equal(out.cpu().numpy(), oracle.fill_outputs_fc(W.numpy(), ridx, B, O, T, E))
     assert np.all(np.isfinite(rxg))
     xg_close(xg.cpu().numpy(), rxg, B, I, T, (O + 31) // 32)
+
+
+# B, T, Nc, O, dgs: fewer columns than a quad; a quad that crosses the row's end
+# in the first, a middle and the last slice; a lone block; a last block of one
+# table; block sizes around the 16 rows in flight; more blocks than a chunk of
+# LDS holds (O = 250: 33 blocks of 252 columns); 512 rows a table
+@pytest.mark.parametrize("ordered", [False, True])
+@pytest.mark.parametrize("B,T,Nc,O,dgs", [(1, 40, 3, 1, 32), (2, 33, 2, 3, 32), (3, 16, 4, 5, 32),
+                                          (70, 97, 3, 30, 32), (5, 64, 3, 259, 16), (300, 80, 3, 250, 2),
+                                          (9, 35, 9, 67, 17), (1, 300, 2, 1030, 1), (2, 5, 2, 4100, 32), (257, 12, 4, 6, 15)])
+def test_forward_blocks(oracle, cuda_device, B, T, Nc, O, dgs, ordered):
+    """Bit-exact for fp32 and int32 sums and for int8 tables, with or without
+    ordered sums."""
+    I, E = 32, 1 << Nc
+    x, anchors, W, _ = make_inputs(B + T, B, I, T, Nc, O)
+    q = torch.randint(-127, 128, (T * E * O,), dtype=torch.int8, generator=torch.Generator().manual_seed(O))
+    scales = torch.rand(T, generator=torch.Generator().manual_seed(T)) * 0.01
+    Wq = (scales[:, None] * q.view(T, -1).float()).reshape(-1)
+    ridx, _, _ = oracle.check_detectors(x.numpy(), anchors.numpy(), B, I, T, Nc)
+    dev = torch.device("cuda:0")
+    for rescaler in (None, 0.5):
+        dm = make_dm(I, O, T, Nc, bgs=dgs, int_rescaler=rescaler)
+        dm.set_ordered_sums(ordered)
+        for tables, call in ((W, lambda *a: dm.forward_step(W.to(dev), *a)),
+                             (Wq, lambda *a: dm.forward_step_i8(q.to(dev), scales.to(dev), *a))):
+            out = torch.zeros(B * O, device=dev)
+            idx = torch.empty(B * T, dtype=torch.int32, device=dev)
+            print(f"[blocks] B={B} T={T} O={O} dgs={dgs} int={rescaler}", flush=True)
+            call(B, x.to(dev), anchors.to(dev), out, idx)
+            want = oracle.fill_outputs_fc(tables.numpy(), ridx, B, O, T, E, dgs=dgs,
+                                          int_mode=rescaler is not None, int_rescaler=rescaler or 1.0)
+            if rescaler is not None:
+                oracle.convert_int_to_float(want, rescaler)
+            assert np.array_equal(idx.cpu().numpy(), ridx)
+            assert np.array_equal(out.cpu().numpy(), want)
