@@ -235,20 +235,7 @@ struct RowLoad<int8_t, 4> {
     }
 };
 
-// Column slices and XCDs.  A launch covers the outputs in `n_slices` slices of
-// 64*VEC columns; workgroup i works on slice i % n_slices.  The hardware hands
-// workgroup i to XCD i % 8, so with 8 (or 16) slices every XCD owns whole
-// slices and sees every sample's accesses to them: table rows (forward,
-// propagate) and gradient rows (weight gradient) are then re-used from that
-// XCD's L2 instead of being fetched once per sample from HBM.
 constexpr int kWPB = kBlock / kWave;  // wavefronts per workgroup
-
-// Floats per lane such that the slices number at least 8 (one per XCD).
-uint32_t pick_vec(uint32_t n_outputs) {
-    if (n_outputs % 4 == 0 && n_outputs >= 64u * 4u * 8u) return 4;
-    if (n_outputs % 2 == 0 && n_outputs >= 64u * 2u * 8u) return 2;
-    return 1;
-}
 
 // Forward gather-sum.  A workgroup owns a sample's column slice, a thread VEC
 // columns of one block of dgs tables at a time (16 rows in flight, fp64,
@@ -280,6 +267,9 @@ __device__ __forceinline__ void load_columns(const WT *p, float *v) {
         const f32x4u q = *reinterpret_cast<const f32x4u *>(p);
 #pragma unroll
         for (int i = 0; i < 4; i++) v[i] = q[i];
+    } else if constexpr (VEC == 2 && sizeof(WT) == 4) {
+        v[0] = p[0];
+        v[1] = p[1];
     } else {
         RowLoad<WT, VEC>::load(p, v);
     }
@@ -971,10 +961,9 @@ struct CvLoad<4> {
     }
 };
 
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// Non-temporal store of VEC floats (one instruction).
+// Non-temporal store of VEC floats (one instruction, 4-byte aligned).
 template <int VEC>
 struct NtStore;
 template <>
@@ -984,34 +973,38 @@ struct NtStore<1> {
 template <>
 struct NtStore<2> {
     __device__ static void store(float *p, const float *v) {
-        __builtin_nontemporal_store(f32x2{v[0], v[1]}, reinterpret_cast<f32x2 *>(p));
+        __builtin_nontemporal_store(f32x2u{v[0], v[1]}, reinterpret_cast<f32x2u *>(p));
     }
 };
 template <>
 struct NtStore<4> {
     __device__ static void store(float *p, const float *v) {
-        __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4 *>(p));
+        __builtin_nontemporal_store(f32x4u{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4u *>(p));
     }
 };
 
 // Table-major weight gradient over column slices.  Wavefront = `rpw` (<= 63)
-// consecutive rows of one table x one column slice (slice -> XCD, so each XCD
-// only ever reads its own column slice of the commit values, which stays in its
-// L2).  The rows' buckets are contiguous in the table's sorted sample list, so
-// the wavefront walks that list in batches of KB samples (the next batch
-// loading while the current one is added, ping-pong) and closes a row whenever
-// the walk crosses its bucket end.  Within a row the commit values are added in
-// ascending sample order into an fp32 (or int32) sum starting from the target
-// value (or zero when overwriting): the reference CPU path's order, so the
-// result is bit-identical to it, and each target element is written exactly
-// once with no atomics.  Commit-value rows are read with buffer loads whose row
-// offset is a scalar register, so a sample costs VEC adds and one lane read.
+// consecutive rows of one table x one column slice; workgroup i works on slice
+// i % n_slices, so that an XCD's L2 holds only the slices' commit values that it
+// re-reads.  The rows' buckets are contiguous in the table's sorted sample list:
+// the wavefront walks that list in batches of KB samples (the next batch loading
+// while the current one is added, ping-pong) and closes a row whenever the walk
+// crosses its bucket end.  Within a row the commit values are added in ascending
+// sample order into an fp32 (or int32) sum starting from the target value (or
+// zero when overwriting): the reference CPU path's order, so the result is
+// bit-identical to it, and each target element is written exactly once with no
+// atomics.  Rows without samples are left alone when accumulating fp32.
+// Commit-value rows are read with buffer loads whose row offset is a scalar
+// register, so a sample costs VEC adds and one lane read.
+//
+// A lane whose columns would cross the row's end reads the row's last VEC
+// columns instead and stores those that are its own.
 template <int VEC, int KB, bool INT_MODE, bool OVERWRITE>
 __global__ __launch_bounds__(kBlock) void k_wgrad_slices(
     const uint32_t *__restrict__ cv, const int32_t *__restrict__ offsets,
     const int32_t *__restrict__ samples, float *__restrict__ target, uint32_t batch,
-    uint32_t n_outputs, uint32_t n_entries, uint32_t n_detectors, uint32_t n_slices, uint32_t rpw,
-    double int_rescaler) {
+    uint32_t n_outputs, uint32_t n_entries, uint32_t n_detectors, uint32_t n_slices, uint32_t lanes,
+    uint32_t rpw, double int_rescaler) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = uniform(threadIdx.x / kWave);
     const uint32_t slice = blockIdx.x % n_slices;
@@ -1021,9 +1014,10 @@ __global__ __launch_bounds__(kBlock) void k_wgrad_slices(
     if (t64 >= n_detectors) return;
     const uint32_t t = (uint32_t)t64;
     const uint32_t e0 = (uint32_t)(unit % groups) * rpw;
-    const uint32_t c = (slice * kWave + lane) * VEC;
-    const bool active = c < n_outputs;
-    const uint32_t cc = active ? c : 0u;
+    const uint32_t c = (slice * lanes + lane) * VEC;
+    const bool active = lane < lanes && c < n_outputs;
+    const uint32_t cc = active ? min(c, n_outputs - VEC) : 0u;
+    const uint32_t own = active ? c - cc : (uint32_t)VEC;  // first of the VEC columns to store
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void *)cv, (short)0, (int)(batch * n_outputs * 4u), 0x00020000);
     const uint32_t voff = cc * 4u;
@@ -1036,6 +1030,9 @@ __global__ __launch_bounds__(kBlock) void k_wgrad_slices(
     float *tb = target + ((size_t)t * n_entries + e0) * n_outputs + cc;
     const int32_t kbeg = __builtin_amdgcn_readfirstlane(offv);
     const int32_t kend = __builtin_amdgcn_readlane(offv, rpw);
+    // a row is opened where it starts, or, accumulating fp32, at its first sample
+    constexpr bool kAll = OVERWRITE || INT_MODE;
+    if (!kAll && kbeg == kend) return;
 
     uint32_t acc[VEC];
     auto init = [&](uint32_t e) {
@@ -1043,7 +1040,7 @@ __global__ __launch_bounds__(kBlock) void k_wgrad_slices(
         for (int q = 0; q < VEC; q++) acc[q] = 0u;  // +0.0f / int 0
         if (!OVERWRITE) {
             float v[VEC];
-            RowLoad<float, VEC>::load(tb + (size_t)e * n_outputs, v);
+            load_columns<float, VEC>(tb + (size_t)e * n_outputs, v);
 #pragma unroll
             for (int q = 0; q < VEC; q++) acc[q] = __float_as_uint(v[q]);
         }
@@ -1051,19 +1048,24 @@ __global__ __launch_bounds__(kBlock) void k_wgrad_slices(
     // the rows are written once and not re-read here: non-temporal stores keep
     // them from evicting the commit values this XCD re-reads from its L2
     auto store = [&](uint32_t e) {
-        if (!active) return;
         float *p = tb + (size_t)e * n_outputs;
         float v[VEC];
 #pragma unroll
         for (int q = 0; q < VEC; q++)
             v[q] = INT_MODE ? (float)(((double)(int32_t)acc[q] * kDenom32Reciproc) / int_rescaler)
                             : __uint_as_float(acc[q]);
-        NtStore<VEC>::store(p, v);
+        if (own == 0)
+            NtStore<VEC>::store(p, v);
+        else
+#pragma unroll
+            for (int q = 1; q < VEC; q++)
+                if (q >= (int)own) NtStore<1>::store(p + q, v + q);
     };
 
     uint32_t e = 0;
     int32_t row_end = __builtin_amdgcn_readlane(offv, 1);
-    init(0);
+    bool open = kAll;
+    if (kAll) init(0);
     for (int32_t k = kbeg; k < kend; k += kWave) {
         const int32_t n = min((int32_t)kWave, kend - k);
         const int32_t idv = smp[k + min((int32_t)lane, n - 1)];
@@ -1081,10 +1083,15 @@ __global__ __launch_bounds__(kBlock) void k_wgrad_slices(
                 if (j0 + j >= n) break;
                 const int32_t kk = k + j0 + j;
                 while (kk >= row_end) {
-                    store(e);
+                    if (kAll || open) store(e);
                     e++;
                     row_end = __builtin_amdgcn_readlane(offv, e + 1);
+                    if (kAll) init(e);
+                    open = false;
+                }
+                if (!kAll && !open) {
                     init(e);
+                    open = true;
                 }
 #pragma unroll
                 for (int q = 0; q < VEC; q++) {
@@ -1109,6 +1116,10 @@ __global__ __launch_bounds__(kBlock) void k_wgrad_slices(
             j0 += KB;
             if (!more_a) break;
         }
+    }
+    if (!kAll) {
+        store(e);  // the row of the last sample
+        return;
     }
     for (;;) {
         store(e);
@@ -1308,13 +1319,23 @@ hipError_t launch_wgrad_fc(const FcShape &s, const float *g, const int32_t *idx,
                                              s.n_entries <= 256 ? key_t : nullptr, key_pitch,
                                              key_shift);
         if (e != hipSuccess) return e;
-        // 4 columns per lane once that still leaves 4 slices (two XCDs per slice)
-        const uint32_t vec = (s.n_outputs % 4 == 0 && s.n_outputs >= 1024) ? 4 : pick_vec(s.n_outputs);
-        const uint32_t n_slices = (s.n_outputs + kWave * vec - 1) / (kWave * vec);
-        // rows a wavefront: 32, or fewer where few tables would leave the grid
-        // short of 16 wavefronts a CU (a feed-forward layer's 16 tables)
-        uint32_t rpw = std::min<uint32_t>(s.n_entries, 32);
-        while (rpw > 4 && (uint64_t)n_slices * s.n_detectors * (s.n_entries / rpw) < 4096) rpw /= 2;
+        // 16 bytes a lane once a row fills the wavefront; an odd width's rows too
+        // (B = 255, T = 2048, O = 1000: 600 us, 870 with 4 bytes a lane)
+        const uint32_t vec = s.n_outputs > 128 ? 4 : s.n_outputs > 64 ? 2 : 1;
+        const uint32_t pieces = (s.n_outputs + vec - 1) / vec;
+        const uint32_t n_slices = (pieces + kWave - 1) / kWave;
+        const uint32_t lanes = (pieces + n_slices - 1) / n_slices;
+        // Rows a wavefront.  With few samples a row the writes bound the kernel, and
+        // they run fastest when the grid writes the gradient in order, few rows a
+        // workgroup (B = 256, T = 4096, E = 256, O = 256: 168 us at 4 rows, 213 at 32;
+        // B = 128, O = 1024: 343 against 445).  From four samples a row the walk
+        // bounds it, which a longer list amortises (B = 1024, T = 8192, O = 1024: 1698
+        // us at 32, 1924 at 4); so do lists of a few samples among untouched rows.
+        const bool walk = s.batch >= 4 * s.n_entries || (!overwrite && !int_mode);
+        // int32 rows cost a conversion each: 8 (B = 256, T = 1024, O = 256: 57 us, 66 at 4).
+        // Fewer again where few tables would leave the grid short of 32 wavefronts a CU.
+        uint32_t rpw = std::min<uint32_t>(s.n_entries, walk ? 32 : int_mode ? 8 : 4);
+        while (rpw > 4 && (uint64_t)n_slices * s.n_detectors * (s.n_entries / rpw) < 8192) rpw /= 2;
         const uint64_t units = (uint64_t)s.n_detectors * (s.n_entries / rpw);
         const uint64_t grid = (uint64_t)n_slices * ((units + kWPB - 1) / kWPB);
         if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
@@ -1330,7 +1351,7 @@ hipError_t launch_wgrad_fc(const FcShape &s, const float *g, const int32_t *idx,
 #define SPIKY_WG(V, IM, OW)                                                                       \
     hipLaunchKernelGGL((k_wgrad_slices<V, 8, IM, OW>), dim3((uint32_t)grid), dim3(kBlock), 0, st, \
                        cv, offsets, samples, target, s.batch, s.n_outputs, s.n_entries,           \
-                       s.n_detectors, n_slices, rpw, int_rescaler)
+                       s.n_detectors, n_slices, lanes, rpw, int_rescaler)
 #define SPIKY_WG_V(IM, OW)                     \
     switch (vec) {                             \
         case 4: SPIKY_WG(4, IM, OW); break;    \

@@ -87,3 +87,41 @@ def test_forward_blocks(oracle, cuda_device, B, T, Nc, O, dgs, ordered):
                 oracle.convert_int_to_float(want, rescaler)
             assert np.array_equal(idx.cpu().numpy(), ridx)
             assert np.array_equal(out.cpu().numpy(), want)
+
+
+# B, T, Nc, O: rows of a lane, of a piece and of a slice and one output more or
+# less (1, 2 and 4 outputs a lane; 256 a slice); one to many samples a row
+@pytest.mark.parametrize("int_rescaler", [None, 0.5])
+@pytest.mark.parametrize("B,T,Nc,O", [(1, 3, 1, 1), (5, 7, 2, 65), (9, 11, 5, 127), (300, 6, 3, 129),
+                                      (70, 9, 6, 257), (33, 5, 7, 255), (140, 40, 2, 514), (6, 70, 8, 131)])
+def test_weight_gradient_rows(oracle, cuda_device, B, T, Nc, O, int_rescaler):
+    """Overwritten and accumulated gradients (run_fc checks both, bit for bit)."""
+    run_fc(oracle, B, 24, T, Nc, O, seed=B * O, int_rescaler=int_rescaler)
+
+
+@pytest.mark.parametrize("O", [10, 129, 300])
+def test_weight_gradient_accumulates(oracle, cuda_device, O):
+    """fp32 accumulation into other values: rows with samples are summed from
+    them in ascending order, rows without keep every bit (negative zeros, NaN)."""
+    B, I, T, Nc = 20, 30, 13, 7
+    E = 1 << Nc
+    x, anchors, W, go = make_inputs(9, B, I, T, Nc, O)
+    before = torch.randn(T * E * O, generator=torch.Generator().manual_seed(3))
+    before[::7] = -0.0
+    ridx, _, _ = oracle.check_detectors(x.numpy(), anchors.numpy(), B, I, T, Nc)
+    free = np.ones((T, E), bool)
+    for t in range(T):
+        free[t, ridx.reshape(B, T)[:, t]] = False
+    before.view(T, E, O)[torch.from_numpy(free)][:, 1:2] = float("nan")
+    dm = make_dm(I, O, T, Nc)
+    dev = torch.device("cuda:0")
+    xd, ad, Wd, gd, wg = (v.to(dev) for v in (x, anchors, W, go, before))
+    out, xg = torch.zeros(B * O, device=dev), torch.zeros(B * I, device=dev)
+    idx = torch.empty(B * T, dtype=torch.int32, device=dev)
+    md, mi = torch.empty(B * T, device=dev), torch.empty(B * T, dtype=torch.int32, device=dev)
+    print(f"[wgrad] accumulate O={O}", flush=True)
+    dm.forward_step(Wd, B, xd, ad, out, idx, 0.0, None, md, mi)
+    dm.backward_backprop(Wd, B, gd, ad, idx, md, mi, xg, -1.0, wg, None)
+    want = before.numpy().copy()
+    oracle.gather_wgrad_fc(go.numpy(), ridx, want, B, O, T, E)
+    assert np.array_equal(wg.cpu().numpy().view(np.int32), want.view(np.int32))
