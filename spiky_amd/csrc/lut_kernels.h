@@ -166,7 +166,7 @@ hipError_t launch_fill_tm_i8(const FcShape &s, const int8_t *q8, const float *sc
 
 // fp32-summation min-margin input gradient through per-slice partial dots.
 // out[i] (+)= sum over k of part[k][i] in ascending k (fp32, or wrapping int32
-// then the int epilogue), i < n, n % 4 == 0.
+// then the int epilogue), i < n.
 hipError_t launch_block_commit(const uint32_t *part, float *out, uint64_t n, uint32_t n_blocks,
                                bool int_mode, double int_rescaler, hipStream_t st);
 bool tm_propagate_applies(const FcShape &s);

@@ -12,10 +12,15 @@
 //                       positional embedding and its min-|value| dimension.
 //   k_seq_pack          idx / mi / md -> one 8-byte record per (t, b, s), so a
 //                       wavefront's walk over positions reads contiguous memory.
-//   k_fill_seq          one wavefront per (sample, later position j, column
-//                       slice): tables in ascending order, pairs i < j summed in
-//                       fp64 and committed once per table -- the reference CPU
-//                       path's order, so the output is bit-identical to it.
+//   k_fill_seq_rows     one wavefront per (table, sample, later position j): its
+//                       pairs i < j summed in fp64 in ascending i from rows read
+//                       where they are, one commit value a table to a partial
+//                       that is added in table order -- the reference CPU path's
+//                       order, so the output is bit-identical to it.
+//   k_fill_seq_lds      the same with the (table, Q) sub-table's column slice in
+//                       LDS, for many pairs a row.
+//   k_fill_seq          the same with the tables walked by the wavefront itself,
+//                       where the partials would not fit.
 //   k_propagate_seq     fp32 summation: one wavefront per (sample, table, j); for
 //                       8 pairs at a time it reads the main, flipped and
 //                       PE-flipped rows, reduces the dots with a DPP
@@ -259,6 +264,134 @@ __global__ __launch_bounds__(kBlock) void k_fill_seq(
         ob[v] = INT_MODE ? (float)(((double)irun[v] * kDenom32Reciproc) / int_rescaler) : run[v];
 }
 
+// The same sums, a wavefront an item: lane l holds VEC columns of one (table,
+// sample, later position j) and adds the item's rows in ascending i in fp64,
+// reading each row where it is in memory, 16 rows in flight; the commit values
+// go to per-table partials that k_fill_commit adds in table order.  Narrow rows
+// (n_outputs <= 128) share a wavefront between items.
+//
+// Items are taken in the bucket sort's order (table, then Q), an eighth of each
+// table's items on every XCD, so that items that read one sub-table run side by
+// side.  What bounds it is the row traffic, which is less than the whole table's
+// only while an item's rows are mostly its own: see seq_fill_by_rows.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int VEC, bool WIDE, bool INT_MODE>
+__global__ __launch_bounds__(kBlock) void k_fill_seq_rows(
+    const float *__restrict__ w, const uint2 *__restrict__ pack, const uint2 *__restrict__ ppack,
+    const int32_t *__restrict__ samples, uint32_t *__restrict__ part, uint32_t batch, uint32_t seq,
+    uint32_t n_outputs, uint32_t n_detectors, uint32_t n_anchors, uint32_t pe_dim, uint32_t lanes,
+    uint32_t n_slices, uint32_t seg_units, double int_rescaler) {
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = uniform(threadIdx.x / kWave);
+    const uint32_t n_rows = batch * seq;
+    // workgroup i runs on XCD i % 8: a table's items in 8 segments, one an XCD
+    const uint32_t xcd = blockIdx.x % 8u, local = blockIdx.x / 8u;
+    const uint32_t slice = local % n_slices;
+    const uint32_t t = local / n_slices / seg_units;
+    const uint32_t per_wave = WIDE ? 1u : kWave / lanes;
+    const uint32_t seg = seg_units * kWPB * per_wave;  // items of a segment
+    const uint32_t g = WIDE ? 0u : lane / lanes, cl = WIDE ? lane : lane % lanes;
+    const uint32_t p = xcd * seg + (local / n_slices % seg_units * kWPB + wave) * per_wave + g;
+    const uint32_t col = (slice * lanes + cl) * VEC;
+    const bool item = g < per_wave && p < min(n_rows, (xcd + 1) * seg);
+    const bool on = item && cl < lanes && col < n_outputs;
+    const uint32_t cs = on ? min(col, n_outputs - VEC) : 0u;
+    const uint32_t row = (uint32_t)samples[(size_t)t * n_rows + min(p, n_rows - 1)];
+    const uint32_t b = row / seq;
+    const uint32_t j = on ? row % seq : 0u;
+    const uint32_t sub_rows = 1u << (n_anchors + pe_dim);
+    const uint2 *kp = pack + (size_t)t * n_rows + (size_t)b * seq;
+    const uint2 *pp = ppack + (size_t)t * (seq - 1);
+    const uint32_t q = rec_idx(kp[row - b * seq]) & ((1u << n_anchors) - 1);
+    const float *sub = w + ((size_t)t * (1u << n_anchors) + q) * sub_rows * n_outputs;
+    auto pair_row = [&](uint32_t i) {
+        return ((rec_idx(kp[i]) << pe_dim) | rec_idx(pp[j - i - 1])) & (sub_rows - 1);
+    };
+
+    double acc[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; v++) acc[v] = 0.0;
+    constexpr int U = 8;
+    float va[U][VEC], vb[U][VEC];
+    auto add = [&](const float (&v)[U][VEC], uint32_t i0, uint32_t end) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int c = 0; c < VEC; c++) acc[c] += i0 + u < end ? (double)v[u][c] : 0.0;
+    };
+    if (WIDE) {
+        // one item a wavefront: its position is uniform, and 64 pairs' row offsets
+        // are formed by 64 lanes and read back lane by lane as scalars
+        const uint32_t ju = uniform(item ? row % seq : 0u);
+        const uint32_t qu = uniform(q);
+        const float *subu = w + ((size_t)t * (1u << n_anchors) + qu) * sub_rows * n_outputs;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)subu, (short)0, (int)(sub_rows * n_outputs * 4u), 0x00020000);
+        const uint32_t voff = cs * 4u;
+        for (uint32_t i0 = 0; i0 < ju; i0 += kWave) {
+            const uint32_t n = min((uint32_t)kWave, ju - i0);
+            const uint32_t i = i0 + min(lane, n - 1);
+            const uint32_t off =
+                (((rec_idx(kp[i]) << pe_dim) | rec_idx(pp[ju - i - 1])) & (sub_rows - 1)) * n_outputs * 4u;
+            auto load = [&](float (&v)[U][VEC], uint32_t k) {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const uint32_t so = (uint32_t)__builtin_amdgcn_readlane((int)off, (int)min(k + u, n - 1));
+                    if constexpr (VEC == 4) {
+                        const u32x4s x = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, so, 0);
+#pragma unroll
+                        for (int c = 0; c < 4; c++) v[u][c] = __uint_as_float(x[c]);
+                    } else {
+                        v[u][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, voff, so, 0));
+                    }
+                }
+            };
+            load(va, 0);
+            for (uint32_t k = 0; k < n; k += 2 * U) {
+                if (k + U < n) load(vb, k + U);
+                add(va, k, n);
+                if (k + 2 * U < n) load(va, k + 2 * U);
+                if (k + U < n) add(vb, k + U, n);
+            }
+        }
+    } else {
+        const float *base = sub + cs;
+        auto load = [&](float (&v)[U][VEC], uint32_t i0) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const float *rp = base + (size_t)pair_row(min(i0 + u, j - 1)) * n_outputs;
+                if constexpr (VEC == 4) {
+                    const f32x4u x = *reinterpret_cast<const f32x4u *>(rp);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) v[u][c] = x[c];
+                } else {
+                    v[u][0] = *rp;
+                }
+            }
+        };
+        for (uint32_t i0 = 0; i0 < j; i0 += 2 * U) {
+            load(va, i0);
+            if (i0 + U < j) load(vb, i0 + U);
+            add(va, i0, j);
+            if (i0 + U < j) add(vb, i0 + U, j);
+        }
+    }
+    if (!on) return;
+    uint32_t *dst = part + ((size_t)t * n_rows + row) * n_outputs + cs;
+    uint32_t o[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; v++)
+        o[v] = INT_MODE ? (uint32_t)(int32_t)(acc[v] * kDenom32 * int_rescaler)
+                        : __float_as_uint((float)acc[v]);
+    if constexpr (VEC == 4)
+        __builtin_nontemporal_store(u32x4u{o[0], o[1], o[2], o[3]}, reinterpret_cast<u32x4u *>(dst));
+    else
+        __builtin_nontemporal_store(o[0], dst);
+}
+
 // ---------------------------------------------------------------------------
 // Sub-table-major forward: one 1024-thread workgroup per (table t, Q value q,
 // column slice of C columns).  The sub-table slice W[t][q][*][c0, c0 + C)
@@ -401,8 +534,16 @@ __global__ __launch_bounds__(kSfThreads) void k_fill_seq_lds(
     while (((seq - 1) >> jsh) >= (uint32_t)kSfLenClasses) jsh++;
     const uint32_t half = lane / L, cl = lane % L;
     uint32_t *my_rows = rowtab + (wave * kSlots + half) * C;
-    const uint32_t slice = blockIdx.x % n_slices;
-    const uint32_t tq = order ? order[blockIdx.x / n_slices] : blockIdx.x / n_slices;  // largest first
+    // a bucket's slices run side by side on one XCD (workgroup i runs on XCD
+    // i % 8), so that its 1 KiB rows are fetched whole (config-5 attention layer:
+    // 2.73 -> 2.63 ms, and 1.50 -> 1.38 ms at an eighth of its batch)
+    uint32_t slice = blockIdx.x % n_slices, rank = blockIdx.x / n_slices;
+    if (gridDim.x % (8u * n_slices) == 0) {
+        const uint32_t local = blockIdx.x / 8u;
+        slice = local % n_slices;
+        rank = local / n_slices * 8u + blockIdx.x % 8u;
+    }
+    const uint32_t tq = order ? order[rank] : rank;  // largest first
     const uint32_t n_q = 1u << n_anchors;
     const uint32_t t = tq / n_q, q = tq % n_q;
     const uint32_t sub_rows = 1u << (n_anchors + pe_dim);
@@ -2284,6 +2425,11 @@ uint64_t seq_tri_bytes(const SeqShape &s) {
 }
 
 // The pair-parallel main pass and its triangle reduction apply (fp32 sums).
+bool seq_partials_fit(const SeqShape &s) {
+    const uint64_t rows = (uint64_t)s.batch * s.seq;
+    return rows <= 0x7fffffffull && (uint64_t)s.n_detectors * rows * s.n_outputs * 4 <= (8ull << 30);
+}
+
 bool seq_pairs_applies(const SeqShape &s) {
     return s.n_outputs % 4 == 0 && s.n_outputs <= (uint32_t)kPairMaxO && seq_tri_bytes(s) <= (16ull << 30);
 }
@@ -2304,15 +2450,26 @@ int seq_grp_bits(const SeqShape &s) {
 // widest power of two <= 64 whose sub-table slice fits the LDS table.
 uint32_t seq_fill_cols(const SeqShape &s) {
     const uint64_t sub_rows = 1ull << (s.n_anchors + s.pe_dim);
-    const uint64_t rows = (uint64_t)s.batch * s.seq;
-    if (s.n_outputs % 4 != 0 || s.seq - 1 > (uint32_t)kSfPe || rows > 0x7fffffffull ||
-        (uint64_t)s.n_detectors * rows * s.n_outputs * 4 > (8ull << 30))
-        return 0;
+    if (s.n_outputs % 4 != 0 || s.seq - 1 > (uint32_t)kSfPe || !seq_partials_fit(s)) return 0;
     uint32_t cols = 64;
     while (cols > 8 && sub_rows * cols > (uint64_t)kSfTabFloats) cols /= 2;
     if (sub_rows * cols > (uint64_t)kSfTabFloats) return 0;
     while (cols > 8 && cols / 2 >= s.n_outputs) cols /= 2;
     return cols;
+}
+
+// The forward reads rows where they are (k_fill_seq_rows) rather than staging
+// every (table, Q) sub-table in LDS while the causal pairs select a table's rows
+// up to three times on average.  T = 64, 65536 rows a table, O = 256, S = 256, rows
+// against staging: 350 / 1210 us at half a pair a row, 1010 / 1380 at two, 1400 /
+// 1440 at three, 1680 / 1480 at four, 3630 / 2630 at sixteen.  Rows too where the
+// staging does not apply (odd widths: B = 32, 16384 rows, O = 255: 3170 us, 17360
+// with a wavefront an output row, k_fill_seq).
+bool seq_fill_by_rows(const SeqShape &s) {
+    const uint64_t sub_rows = 1ull << (s.n_anchors + s.pe_dim);
+    if (!seq_partials_fit(s) || sub_rows * s.n_outputs * 4 > 0x7fffffffull) return false;
+    const uint64_t pairs = (uint64_t)s.batch * s.seq * (s.seq - 1) / 2;
+    return pairs <= 3 * (sub_rows << s.n_anchors) || seq_fill_cols(s) == 0;
 }
 
 // Columns of a weight-gradient slice (0: the sort path does not apply): a
@@ -2370,7 +2527,8 @@ hipError_t launch_forward_seq(const SeqShape &s, const float *w, const float *x,
                               float cmp_eps, bool int_mode, double int_rescaler, Scratch &scratch,
                               hipStream_t st) {
     const uint32_t rows = s.batch * s.seq;
-    const uint32_t fcols = seq_fill_cols(s);
+    const bool by_rows = seq_fill_by_rows(s);
+    const uint32_t fcols = by_rows ? 0 : seq_fill_cols(s);
     // scratch: packed keys [T][B*S] | positional keys [T][S-1] | and for the
     // LDS-sliced forward: bucket offsets [T][2^Nc+1] | samples [T][B*S] |
     // per-table partials [T][B*S][O]
@@ -2379,7 +2537,7 @@ hipError_t launch_forward_seq(const SeqShape &s, const float *w, const float *x,
     uint2 *ppack = lay.take<uint2>((size_t)s.n_detectors * (s.seq - 1) * 8);
     int32_t *offsets = nullptr, *samples = nullptr;
     uint32_t *part = nullptr, *order = nullptr;
-    if (fcols > 0) {
+    if (by_rows || fcols > 0) {
         offsets = lay.take<int32_t>((size_t)s.n_detectors * ((1u << s.n_anchors) + 1) * 4);
         samples = lay.take<int32_t>((size_t)s.n_detectors * rows * 4);
         part = lay.take<uint32_t>((size_t)s.n_detectors * rows * s.n_outputs * 4);
@@ -2407,10 +2565,38 @@ hipError_t launch_forward_seq(const SeqShape &s, const float *w, const float *x,
                        (const int32_t *)nullptr, ppack, s.seq - 1, s.n_detectors);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (fcols > 0) {
-        FcShape fs2 = fs;
-        e = launch_bucket_samples(fs2, idx, offsets, samples, st);
+    if (by_rows || fcols > 0) {
+        e = launch_bucket_samples(fs, idx, offsets, samples, st);
         if (e != hipSuccess) return e;
+    }
+    if (by_rows) {
+        const uint32_t vec = s.n_outputs >= 4 ? 4 : 1;
+        const uint32_t pieces = (s.n_outputs + vec - 1) / vec;
+        const uint32_t n_slices = (pieces + kWave - 1) / kWave;
+        const uint32_t lanes = (pieces + n_slices - 1) / n_slices;
+        const bool wide = lanes > kWave / 2;
+        const uint32_t per_wg = kWPB * (wide ? 1 : kWave / lanes);
+        const uint32_t seg_units = ((rows + 7) / 8 + per_wg - 1) / per_wg;
+        const uint64_t grid = 8ull * seg_units * n_slices * s.n_detectors;
+        if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
+#define SPIKY_FROWS(V, WD, IM)                                                                     \
+    hipLaunchKernelGGL((k_fill_seq_rows<V, WD, IM>), dim3((uint32_t)grid), dim3(kBlock), 0, st, w,  \
+                       pack, ppack, samples, part, s.batch, s.seq, s.n_outputs, s.n_detectors,      \
+                       s.n_anchors, s.pe_dim, lanes, n_slices, seg_units, int_rescaler)
+        if (vec == 1) {
+            if (int_mode) SPIKY_FROWS(1, false, true); else SPIKY_FROWS(1, false, false);
+        } else if (wide) {
+            if (int_mode) SPIKY_FROWS(4, true, true); else SPIKY_FROWS(4, true, false);
+        } else {
+            if (int_mode) SPIKY_FROWS(4, false, true); else SPIKY_FROWS(4, false, false);
+        }
+#undef SPIKY_FROWS
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        return launch_block_commit(part, out, (uint64_t)rows * s.n_outputs, s.n_detectors, int_mode,
+                                   int_rescaler, st);
+    }
+    if (fcols > 0) {
         const uint32_t n_slices = (s.n_outputs + fcols - 1) / fcols;
         const uint64_t grid = (uint64_t)s.n_detectors * (1u << s.n_anchors) * n_slices;
         if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;

@@ -609,6 +609,32 @@ __global__ __launch_bounds__(256) void k_fill_commit(const uint32_t *__restrict_
     *op = run;
 }
 
+// The same a word at a time, for totals that are not whole quads.
+template <bool INT_MODE>
+__global__ __launch_bounds__(256) void k_commit_words(const uint32_t *__restrict__ part,
+                                                      float *__restrict__ out, uint64_t n,
+                                                      uint32_t n_blocks, double int_rescaler) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float run = out[i];
+    int32_t irun = __float_as_int(run);
+    constexpr int kU = 16;
+    for (uint32_t k = 0; k < n_blocks; k += kU) {
+        uint32_t v[kU];
+#pragma unroll
+        for (int u = 0; u < kU; u++) v[u] = part[(uint64_t)min(k + u, n_blocks - 1) * n + i];
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            if (k + u >= n_blocks) break;
+            if (INT_MODE)
+                irun = wrap_add(irun, (int32_t)v[u]);
+            else
+                run += __uint_as_float(v[u]);
+        }
+    }
+    out[i] = INT_MODE ? (float)(((double)irun * kDenom32Reciproc) / int_rescaler) : run;
+}
+
 // ---------------------------------------------------------------------------
 // Propagate partials.  dpart[s][t][b] = fp32(sum over slice s's columns of
 // (W[t][main] - W[t][alt]) * g[b]).  Key = main * 128 | (alt * 128) << 16: the
@@ -1337,7 +1363,17 @@ hipError_t launch_fill_tm_i8(const FcShape &s, const int8_t *q8, const float *sc
 
 hipError_t launch_block_commit(const uint32_t *part, float *out, uint64_t n, uint32_t n_blocks,
                                bool int_mode, double int_rescaler, hipStream_t st) {
-    if (n % 4 != 0) return hipErrorInvalidValue;
+    if (n % 4 != 0) {
+        const uint64_t grid = (n + 255) / 256;
+        if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
+        if (int_mode)
+            hipLaunchKernelGGL(k_commit_words<true>, dim3((uint32_t)grid), dim3(256), 0, st, part, out, n,
+                               n_blocks, int_rescaler);
+        else
+            hipLaunchKernelGGL(k_commit_words<false>, dim3((uint32_t)grid), dim3(256), 0, st, part, out, n,
+                               n_blocks, int_rescaler);
+        return hipGetLastError();
+    }
     const uint64_t n_quads = n / 4;
     const uint64_t cgrid = (n_quads + 255) / 256;
     if (cgrid > 0x7fffffffu) return hipErrorInvalidConfiguration;

@@ -125,3 +125,17 @@ def test_weight_gradient_accumulates(oracle, cuda_device, O):
     want = before.numpy().copy()
     oracle.gather_wgrad_fc(go.numpy(), ridx, want, B, O, T, E)
     assert np.array_equal(wg.cpu().numpy().view(np.int32), want.view(np.int32))
+
+
+# B, S, T, Nc, Npe, O: rows read where they are -- fewer columns than a lane's
+# four, several items a wavefront, a quad over the row's end, a whole wavefront,
+# two slices; one pair, 64 pairs and one more; totals that are not whole quads
+# -- and, from three pairs a row, odd widths and staged slices (whole, partial)
+@pytest.mark.parametrize("int_rescaler", [None, 0.5])
+@pytest.mark.parametrize("B,S,T,Nc,Npe,O", [(1, 2, 3, 4, 2, 1), (3, 17, 5, 3, 3, 3), (2, 9, 9, 4, 0, 33),
+                                            (1, 66, 3, 4, 4, 130), (2, 65, 2, 4, 3, 256),
+                                            (1, 33, 2, 4, 2, 261), (5, 40, 11, 2, 1, 35),
+                                            (6, 40, 8, 2, 1, 64), (6, 40, 3, 2, 2, 36), (4, 70, 2, 1, 0, 8)])
+def test_seq_forward_rows(oracle, cuda_device, B, S, T, Nc, Npe, O, int_rescaler):
+    from test_gpu_seq import run_seq
+    run_seq(oracle, B, S, 20, T, Nc, Npe, O, seed=S + O, int_rescaler=int_rescaler, int_grad=True)
