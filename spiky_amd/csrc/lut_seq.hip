@@ -1352,7 +1352,27 @@ struct GrpItem {
     uint2 ent;
 };
 
-template <int NCH>
+// The sum of a slot's 8 lanes in fp64 (all of them get it).
+__device__ __forceinline__ double grp_sum8d(double v) {
+    v += dpp_f64<0x141>(v);  // half mirror
+    v += dpp_f64<0xB1>(v);   // lane ^ 1
+    v += dpp_f64<0x4E>(v);   // lane ^ 2
+    return v;
+}
+
+// rows of n_outputs floats -> rows of `padded`, zeros past their end
+__global__ __launch_bounds__(kBlock) void k_pad_rows(const float *__restrict__ src, float *__restrict__ dst,
+                                                     uint64_t n, uint32_t n_outputs, uint32_t padded) {
+    const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t c = (uint32_t)(i % padded);
+    dst[i] = c < n_outputs ? src[i / padded * n_outputs + c] : 0.0f;
+}
+
+// PAD: rows of any width up to NCH * 32 outputs (n_outputs), staged with zeros
+// past their end; g then comes padded to NCH * 32 as well, and the dots are
+// summed in fp64 throughout, as the kernels of those widths always have.
+template <int NCH, bool PAD>
 __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
     const float *__restrict__ w, const float *__restrict__ g, const uint2 *__restrict__ pack,
     const uint2 *__restrict__ ppack, const int32_t *__restrict__ offsets,
@@ -1361,8 +1381,11 @@ __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
     const uint32_t *__restrict__ off_a, const uint2 *__restrict__ list_b,
     const uint32_t *__restrict__ off_b, double *__restrict__ macc, double *__restrict__ dpe,
     uint32_t batch, uint32_t seq, uint32_t n_detectors, uint32_t n_anchors, uint32_t pe_dim,
-    uint32_t gb, uint32_t per_xcd) {
+    uint32_t gb, uint32_t per_xcd, uint32_t n_outputs) {
     constexpr uint32_t O = NCH * 32;
+    using Dot = typename std::conditional<PAD, double, float>::type;
+    // the widest fp64 form has registers for one item's g: loaded when the item is taken
+    constexpr bool kOneSet = PAD && NCH == 8;
     constexpr uint32_t kRowBytes = O * 4;
     __shared__ __attribute__((aligned(16))) uint8_t tab[kGrpTabBytes];
     __shared__ double dsum[kGrpMaxDist];
@@ -1392,7 +1415,24 @@ __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
     const uint32_t n_dist = seq - 1;
 
     // stage the group's rows (one contiguous block of the table)
-    {
+    if constexpr (PAD) {
+        const float *src = w + ((((size_t)t << n_anchors | Q) << kbits) | ((size_t)G << (gb + pe_dim))) * n_outputs;
+        const uint32_t n_q = (1u << (gb + pe_dim)) * (O / 4);
+        for (uint32_t e = tid; e < n_q; e += kGrpThreads) {
+            const uint32_t c = e % (O / 4) * 4;
+            const float *rp = src + (size_t)(e / (O / 4)) * n_outputs + c;
+            f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (c + 4 <= n_outputs) {
+                const f32x4u u = *reinterpret_cast<const f32x4u *>(rp);
+                v = f32x4{u[0], u[1], u[2], u[3]};
+            } else {
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+                    if (c + k < n_outputs) v[k] = rp[k];
+            }
+            *reinterpret_cast<f32x4 *>(tab + e * 16) = v;
+        }
+    } else {
         const uint32_t bytes = (1u << (gb + pe_dim)) * kRowBytes;
         const uint8_t *src = reinterpret_cast<const uint8_t *>(
             w + ((((size_t)t << n_anchors | Q) << kbits) | ((size_t)G << (gb + pe_dim))) * O);
@@ -1461,13 +1501,7 @@ __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
             if (lane == 0) v = atomicAdd(&next_item, 1u);
             return uniform(v);  // lane 0 is the first active lane here
         };
-        // an item's loads: g[b][j] in this lane's chunk order and the first
-        // candidate of its lists (main role: lanes 0-31 list A, 32-47 list B;
-        // Q-flip role: every lane list A)
-        auto issue = [&](uint32_t k, uint4 &mm, float (&gg)[NCH][4]) -> uint2 {
-            mm = meta[k];
-            const uint32_t row = mm.x & 0x7FFFFFFu;
-            const bool main_r = c0 + k < n_main;
+        auto load_g = [&](uint32_t row, float (&gg)[NCH][4]) {
             const float *g0 = g + (size_t)row * O + c0l / 4;
             const float *g1 = g + (size_t)row * O + c1l / 4;
 #pragma unroll
@@ -1477,6 +1511,15 @@ __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
 #pragma unroll
                 for (int c = 0; c < 4; c++) gg[kk][c] = v[c];
             }
+        };
+        // an item's loads: g[b][j] in this lane's chunk order and the first
+        // candidate of its lists (main role: lanes 0-31 list A, 32-47 list B;
+        // Q-flip role: every lane list A)
+        auto issue = [&](uint32_t k, uint4 &mm, float (&gg)[NCH][4]) -> uint2 {
+            mm = meta[k];
+            const uint32_t row = mm.x & 0x7FFFFFFu;
+            const bool main_r = c0 + k < n_main;
+            if (!kOneSet) load_g(row, gg);
             const bool use_b = main_r && lane >= 32;
             const uint32_t rng = use_b ? mm.w : mm.z;
             const uint32_t cur = (rng & 0xFFFFu) + (use_b ? lane - 32 : lane);
@@ -1490,6 +1533,7 @@ __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
         auto visit = [&](const GrpItem cur, float (&gf)[NCH][4], float (&gn)[NCH][4]) -> GrpItem {
             const uint32_t it = cur.it;
             const uint4 m = cur.m;
+            if constexpr (kOneSet) load_g(m.x & 0x7FFFFFFu, gf);
             // wait for this item's loads before the next item's are issued: the
             // counter then covers them alone
 #pragma unroll
@@ -1530,18 +1574,24 @@ __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
                     const bool on = p < n;
                     const uint8_t *t0 = tab + ((e & kEntRow) | c0l);
                     const uint8_t *t1 = tab + ((e & kEntRow) | c1l);
-                    float f0 = 0.f, f1 = 0.f, f2 = 0.f, f3 = 0.f;
+                    Dot f0 = 0, f1 = 0, f2 = 0, f3 = 0;
 #pragma unroll
                     for (int k = 0; k < NCH; k++) {
                         const f32x4 v = (k & 1) ? *reinterpret_cast<const f32x4 *>(t1 + (k - 1) * 128)
                                                 : *reinterpret_cast<const f32x4 *>(t0 + k * 128);
-                        f0 = fmaf(v[0], gf[k][0], f0);
-                        f1 = fmaf(v[1], gf[k][1], f1);
-                        f2 = fmaf(v[2], gf[k][2], f2);
-                        f3 = fmaf(v[3], gf[k][3], f3);
+                        if constexpr (kOneSet)  // g stays fp32: widened in every step, not once for all
+                            __asm__ volatile("" : "+v"(gf[k][0]), "+v"(gf[k][1]), "+v"(gf[k][2]), "+v"(gf[k][3]));
+                        f0 = fma((Dot)v[0], (Dot)gf[k][0], f0);
+                        f1 = fma((Dot)v[1], (Dot)gf[k][1], f1);
+                        f2 = fma((Dot)v[2], (Dot)gf[k][2], f2);
+                        f3 = fma((Dot)v[3], (Dot)gf[k][3], f3);
                     }
-                    const float part = on ? (f0 + f1) + (f2 + f3) : 0.f;
-                    const double tot = (double)grp_sum8f(part);
+                    const Dot part = on ? (f0 + f1) + (f2 + f3) : (Dot)0;
+                    double tot;
+                    if constexpr (PAD)
+                        tot = grp_sum8d(part);
+                    else
+                        tot = (double)grp_sum8f(part);
                     if constexpr (!kMain) {
                         jacc -= tot;  // Q-flip entries: cj = -1, no other share
                     } else {
@@ -1668,16 +1718,20 @@ __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
             return nx;
         };
 
-        float gr0[NCH][4], gr1[NCH][4];
+        float gr0[NCH][4], gr1[kOneSet ? 1 : NCH][4];
         GrpItem cur;
         cur.it = fetch();
         cur.m = make_uint4(0u, 0u, 0u, 0u);
         cur.ent = grp_none();
         if (cur.it < cn) cur.ent = issue(cur.it, cur.m, gr0);
         while (cur.it < cn) {
-            cur = visit(cur, gr0, gr1);
-            if (cur.it >= cn) break;
-            cur = visit(cur, gr1, gr0);
+            if constexpr (kOneSet) {
+                cur = visit(cur, gr0, gr0);
+            } else {
+                cur = visit(cur, gr0, gr1);
+                if (cur.it >= cn) break;
+                cur = visit(cur, gr1, gr0);
+            }
         }
         if (fl_pend) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1910,7 +1964,35 @@ __global__ __launch_bounds__(kSeqWgThreads) void k_bucket_order(const int32_t *_
     for (uint32_t b = tid; b < n_buckets; b += kSeqWgThreads) order[atomicAdd(&hist[cls(b)], 1u)] = b;
 }
 
-template <bool INT_MODE, bool OVERWRITE, bool WIDE>
+// Four words at p of which `left` (>= 1) lie in the row: one 16-byte access, or
+// with ODD (rows that are not whole 16-byte pieces, or not aligned to them) one
+// unaligned access, and single words at the row's end.
+template <bool ODD>
+__device__ __forceinline__ u32x4 load_quad(const uint32_t *p, uint32_t left) {
+    if constexpr (!ODD) return *reinterpret_cast<const u32x4 *>(p);
+    if (left >= 4) {
+        const u32x4u u = *reinterpret_cast<const u32x4u *>(p);
+        return u32x4{u[0], u[1], u[2], u[3]};
+    }
+    u32x4 v = u32x4{p[0], 0u, 0u, 0u};
+    if (left > 1) v[1] = p[1];
+    if (left > 2) v[2] = p[2];
+    return v;
+}
+template <bool ODD>
+__device__ __forceinline__ void store_quad(uint32_t *p, const u32x4 &v, uint32_t left) {
+    if constexpr (!ODD) {
+        *reinterpret_cast<u32x4 *>(p) = v;
+    } else if (left >= 4) {
+        *reinterpret_cast<u32x4u *>(p) = u32x4u{v[0], v[1], v[2], v[3]};
+    } else {
+        p[0] = v[0];
+        if (left > 1) p[1] = v[1];
+        if (left > 2) p[2] = v[2];
+    }
+}
+
+template <bool INT_MODE, bool OVERWRITE, bool WIDE, bool ODD>
 __global__ __launch_bounds__(kSeqWgThreads) void k_wgrad_seq_sort(
     const uint32_t *__restrict__ cv, const int32_t *__restrict__ offsets,
     const int32_t *__restrict__ samples, const uint2 *__restrict__ pack,
@@ -2100,7 +2182,7 @@ __global__ __launch_bounds__(kSeqWgThreads) void k_wgrad_seq_sort(
                     const uint32_t it = (tid >> 4) + 64u * u;
                     pre[u] = u32x4{0u, 0u, 0u, 0u};
                     if (it < nb && cq < n_outputs)
-                        pre[u] = *reinterpret_cast<const u32x4 *>(cv + (size_t)bitems[it] * n_outputs + cq);
+                        pre[u] = load_quad<ODD>(cv + (size_t)bitems[it] * n_outputs + cq, n_outputs - cq);
                 }
             };
             auto gv_store = [&]() {
@@ -2125,8 +2207,8 @@ __global__ __launch_bounds__(kSeqWgThreads) void k_wgrad_seq_sort(
                     whi[u] = u32x4{0u, 0u, 0u, 0u};
                     if (it < nb) {
                         const uint32_t *src = cv + (size_t)bitems[it] * n_outputs + cq;
-                        if (cq < n_outputs) wlo[u] = *reinterpret_cast<const u32x4 *>(src);
-                        if (cq + 64u < n_outputs) whi[u] = *reinterpret_cast<const u32x4 *>(src + 64);
+                        if (cq < n_outputs) wlo[u] = load_quad<ODD>(src, n_outputs - cq);
+                        if (cq + 64u < n_outputs) whi[u] = load_quad<ODD>(src + 64, n_outputs - cq - 64u);
                     }
                 }
             };
@@ -2230,20 +2312,21 @@ __global__ __launch_bounds__(kSeqWgThreads) void k_wgrad_seq_sort(
 #pragma unroll
                                 for (int h = 0; h < 2; h++) {
                                     if (cq + 64u * h >= n_outputs) continue;
-                                    u32x4 *p = reinterpret_cast<u32x4 *>(dst + (size_t)row * n_outputs + cq + 64u * h);
+                                    uint32_t *p = reinterpret_cast<uint32_t *>(dst + (size_t)row * n_outputs + cq + 64u * h);
+                                    const uint32_t left = n_outputs - cq - 64u * h;
                                     u32x4 o;
                                     if (store) {
 #pragma unroll
                                         for (int c = 0; c < 4; c++)
                                             o[c] = INT_MODE ? ai[4 * h + c] : __float_as_uint(af[4 * h + c]);
                                     } else {
-                                        const u32x4 old = *p;
+                                        const u32x4 old = load_quad<ODD>(p, left);
 #pragma unroll
                                         for (int c = 0; c < 4; c++)
                                             o[c] = INT_MODE ? (uint32_t)wrap_add((int32_t)ai[4 * h + c], (int32_t)old[c])
                                                             : __float_as_uint(__uint_as_float(old[c]) + af[4 * h + c]);
                                     }
-                                    *p = o;
+                                    store_quad<ODD>(p, o, left);
                                 }
                             }
                             continue;
@@ -2278,19 +2361,20 @@ __global__ __launch_bounds__(kSeqWgThreads) void k_wgrad_seq_sort(
                             add(gb);
                         }
                         if (have && (store || np > 0) && cq < n_outputs) {
-                            u32x4 *p = reinterpret_cast<u32x4 *>(dst + (size_t)row * n_outputs + cq);
+                            uint32_t *p = reinterpret_cast<uint32_t *>(dst + (size_t)row * n_outputs + cq);
+                            const uint32_t left = n_outputs - cq;
                             u32x4 o;
                             if (store) {
 #pragma unroll
                                 for (int c = 0; c < 4; c++) o[c] = INT_MODE ? ai[c] : __float_as_uint(af[c]);
                             } else {
-                                const u32x4 old = *p;
+                                const u32x4 old = load_quad<ODD>(p, left);
 #pragma unroll
                                 for (int c = 0; c < 4; c++)
                                     o[c] = INT_MODE ? (uint32_t)wrap_add((int32_t)ai[c], (int32_t)old[c])
                                                     : __float_as_uint(__uint_as_float(old[c]) + af[c]);
                             }
-                            *p = o;
+                            store_quad<ODD>(p, o, left);
                         }
                     }
                     // the wide walk's next pass: each wave issues its share of the
@@ -2434,14 +2518,24 @@ bool seq_pairs_applies(const SeqShape &s) {
     return s.n_outputs % 4 == 0 && s.n_outputs <= (uint32_t)kPairMaxO && seq_tri_bytes(s) <= (16ull << 30);
 }
 
+// Outputs of the grouped input-gradient pass's rows in LDS: the next of 64, 128, 256.
+uint32_t seq_grp_width(const SeqShape &s) { return s.n_outputs <= 64 ? 64 : s.n_outputs <= 128 ? 128 : 256; }
+
 // K-group bits of the grouped input-gradient pass (-1: it does not apply):
 // the widest group whose 2^(gb + Npe) rows fit the 128 KiB LDS table.
 int seq_grp_bits(const SeqShape &s) {
-    if (s.n_outputs != 64 && s.n_outputs != 128 && s.n_outputs != 256) return -1;
+    if (s.n_outputs > 256) return -1;
+    // padded rows: up to 128 outputs, odd widths (whose other form is one thread a pair
+    // and block: B = 32, T = 64, O = 255, 16384 rows a table: 214 -> 9 ms), and wider
+    // rows from 16 pairs a row (O = 252: 11.3 -> 9.3 ms with the weight gradient; at
+    // four pairs, B = 1, O = 200, 0.81 against 0.67 ms)
+    if (s.n_outputs > 128 && s.n_outputs != 256 && s.n_outputs % 4 == 0 &&
+        (uint64_t)s.batch * s.seq * (s.seq - 1) / 2 < 16ull << (2 * s.n_anchors + s.pe_dim))
+        return -1;
     if (s.n_anchors > 10 || s.seq < 2 || s.seq - 1 > (uint32_t)kGrpMaxDist) return -1;
     if ((uint64_t)s.batch * s.seq >= (1ull << 27)) return -1;  // rows in 27 bits of the item metadata
     uint32_t lr = 0;
-    while ((kGrpTabBytes >> (lr + 1)) >= (int)(s.n_outputs * 4)) lr++;
+    while ((kGrpTabBytes >> (lr + 1)) >= (int)(seq_grp_width(s) * 4)) lr++;
     if (s.pe_dim > lr) return -1;
     return (int)std::min<uint32_t>(s.n_anchors, lr - s.pe_dim);
 }
@@ -2687,6 +2781,9 @@ hipError_t launch_backward_seq(const SeqShape &s, float *w, const float *g, cons
     uint32_t *wg_order = lay.take<uint32_t>((size_t)s.n_detectors * (1u << s.n_anchors) * 4);
     uint2 *list_a = nullptr, *list_b = nullptr;
     uint32_t *off_a = nullptr, *off_b = nullptr;
+    const uint32_t gw = seq_grp_width(s);
+    const bool pad = gb >= 0 && gw != s.n_outputs;
+    float *gp = pad ? lay.take<float>((size_t)rows * gw * 4) : nullptr;
     if (gb >= 0) {
         const uint64_t tb = (uint64_t)s.n_detectors * s.batch;
         const uint64_t ng = 1ull << (s.n_anchors - gb);
@@ -2723,7 +2820,7 @@ hipError_t launch_backward_seq(const SeqShape &s, float *w, const float *g, cons
 
     // input and positional gradients
     const uint32_t nj = (s.n_outputs + 255) / 256;
-    if (!int_mode && s.n_outputs % 4 == 0 && nj <= 4) {
+    if (gb >= 0 || (!int_mode && s.n_outputs % 4 == 0 && nj <= 4)) {
         const uint64_t n_acc = (uint64_t)rows * s.n_detectors;
         hipLaunchKernelGGL(k_zero64, dim3(blocks_for(n_acc)), dim3(kBlock), 0, st, dq, n_acc);
         hipLaunchKernelGGL(k_zero64, dim3(blocks_for(n_acc)), dim3(kBlock), 0, st, dq_alt, n_acc);
@@ -2754,15 +2851,27 @@ hipError_t launch_backward_seq(const SeqShape &s, float *w, const float *g, cons
             const uint64_t n_wg = (uint64_t)s.n_detectors * (1u << s.n_anchors) * ng;
             const uint64_t per_xcd = (n_wg + 7) / 8;
             if (per_xcd * 8 > 0x7fffffffu) return hipErrorInvalidConfiguration;
-#define SPIKY_PGRP(NCH)                                                                             \
-    hipLaunchKernelGGL(k_propagate_seq_grp<NCH>, dim3((uint32_t)(per_xcd * 8)), dim3(kGrpThreads), \
-                       0, st, w, g, pack, ppack, offsets, samples, offsets2, samples2, list_a,      \
-                       off_a, list_b, off_b, dq, dpe, s.batch, s.seq, s.n_detectors, s.n_anchors,   \
-                       s.pe_dim, (uint32_t)gb, (uint32_t)per_xcd)
-            switch (s.n_outputs) {
-                case 64: SPIKY_PGRP(2); break;
-                case 128: SPIKY_PGRP(4); break;
-                default: SPIKY_PGRP(8); break;
+#define SPIKY_PGRP(NCH, PAD)                                                                        \
+    hipLaunchKernelGGL((k_propagate_seq_grp<NCH, PAD>), dim3((uint32_t)(per_xcd * 8)),              \
+                       dim3(kGrpThreads), 0, st, w, pad ? gp : g, pack, ppack, offsets, samples,    \
+                       offsets2, samples2, list_a, off_a, list_b, off_b, dq, dpe, s.batch, s.seq,   \
+                       s.n_detectors, s.n_anchors, s.pe_dim, (uint32_t)gb, (uint32_t)per_xcd,       \
+                       s.n_outputs)
+            if (pad) {
+                const uint64_t n_gp = (uint64_t)rows * gw;
+                hipLaunchKernelGGL(k_pad_rows, dim3(blocks_for(n_gp)), dim3(kBlock), 0, st, g, gp, n_gp,
+                                   s.n_outputs, gw);
+                switch (gw) {
+                    case 64: SPIKY_PGRP(2, true); break;
+                    case 128: SPIKY_PGRP(4, true); break;
+                    default: SPIKY_PGRP(8, true); break;
+                }
+            } else {
+                switch (gw) {
+                    case 64: SPIKY_PGRP(2, false); break;
+                    case 128: SPIKY_PGRP(4, false); break;
+                    default: SPIKY_PGRP(8, false); break;
+                }
             }
 #undef SPIKY_PGRP
             hipLaunchKernelGGL(k_seq_xgrad, dim3(blocks_for(n_acc)), dim3(kBlock), 0, st, dq,
@@ -2835,8 +2944,10 @@ hipError_t launch_backward_seq(const SeqShape &s, float *w, const float *g, cons
         const uint64_t grid = (uint64_t)s.n_detectors * (1u << s.n_anchors);
         if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
         const uint32_t ipb = seq_wg_items(s, cols);
-        // 16-byte row pieces: 64-column slices of whole quads, 16-byte aligned rows
-        const bool quad = cols == 64 && s.n_outputs % 4 == 0 && ((uintptr_t)target & 15) == 0;
+        // 64-column slices move 16 bytes a lane, also where the rows are not whole
+        // 16-byte pieces or aligned to them (`odd`)
+        const bool quad = cols == 64;
+        const bool odd = s.n_outputs % 4 != 0 || ((uintptr_t)target & 15) != 0;
         // two 64-column slices a pass where the sub-table's row arrays leave LDS room
         const bool wide = quad && (1u << (s.n_anchors + s.pe_dim)) <= (uint32_t)kSeqWgWideRows;
         if (grid <= kOrderMaxBuckets)
@@ -2844,15 +2955,17 @@ hipError_t launch_backward_seq(const SeqShape &s, float *w, const float *g, cons
                                1u << s.n_anchors, (uint32_t)grid, wg_order);
         else
             wg_order = nullptr;
-#define SPIKY_WSEQ(IM, OW, WD)                                                                              \
-    hipLaunchKernelGGL((k_wgrad_seq_sort<IM, OW, WD>), dim3((uint32_t)grid), dim3(kSeqWgThreads), 0, st, cv, \
-                       offsets, samples, pack, ppack, wg_order, target, s.batch, s.seq, s.n_outputs,        \
-                       s.n_detectors, s.n_anchors, s.pe_dim, cols, n_slices, ipb, int_rescaler, quad)
-#define SPIKY_WSEQ_W(IM, OW)           \
-    if (wide)                          \
-        SPIKY_WSEQ(IM, OW, true);      \
-    else                               \
-        SPIKY_WSEQ(IM, OW, false);
+#define SPIKY_WSEQ(IM, OW, WD, ODD)                                                                         \
+    hipLaunchKernelGGL((k_wgrad_seq_sort<IM, OW, WD, ODD>), dim3((uint32_t)grid), dim3(kSeqWgThreads), 0,   \
+                       st, cv, offsets, samples, pack, ppack, wg_order, target, s.batch, s.seq,             \
+                       s.n_outputs, s.n_detectors, s.n_anchors, s.pe_dim, cols, n_slices, ipb,              \
+                       int_rescaler, quad)
+#define SPIKY_WSEQ_W(IM, OW)                                                                 \
+    if (wide) {                                                                              \
+        if (odd) SPIKY_WSEQ(IM, OW, true, true); else SPIKY_WSEQ(IM, OW, true, false);       \
+    } else {                                                                                 \
+        if (odd) SPIKY_WSEQ(IM, OW, false, true); else SPIKY_WSEQ(IM, OW, false, false);     \
+    }
         if (int_mode) {
             if (overwrite) { SPIKY_WSEQ_W(true, true) } else { SPIKY_WSEQ_W(true, false) }
         } else {

@@ -139,3 +139,24 @@ def test_weight_gradient_accumulates(oracle, cuda_device, O):
 def test_seq_forward_rows(oracle, cuda_device, B, S, T, Nc, Npe, O, int_rescaler):
     from test_gpu_seq import run_seq
     run_seq(oracle, B, S, 20, T, Nc, Npe, O, seed=S + O, int_rescaler=int_rescaler, int_grad=True)
+
+
+# S, Npe, O: the grouped input gradient over rows padded to 64, 128 and 256
+# outputs and the weight gradient's unaligned 16-byte pieces: one output, a piece
+# and one more, a slice and one more, two slices less one, widths past 128 at few
+# and at many pairs a row (even widths change form there)
+@pytest.mark.parametrize("B,S,Nc,Npe,O", [(2, 9, 3, 2, 1), (3, 20, 4, 0, 5), (2, 17, 3, 1, 33),
+                                          (2, 30, 3, 3, 65), (1, 40, 3, 2, 127), (3, 25, 4, 0, 129),
+                                          (2, 12, 4, 1, 132), (6, 33, 2, 1, 252), (2, 30, 3, 4, 255)])
+@pytest.mark.parametrize("policy", ["dense", "accumulate", "internal"])
+def test_seq_backward_padded_rows(oracle, cuda_device, B, S, Nc, Npe, O, policy):
+    from test_gpu_seq import run_seq
+    # the accumulating check wants rows that no pair reaches
+    accumulate = policy == "accumulate" and Nc > 2
+    run_seq(oracle, B, S, 24, 3, Nc, Npe, O, seed=O, internal=policy == "internal", accumulate=accumulate)
+
+
+@pytest.mark.parametrize("O", [70, 130])
+def test_seq_int32_unaligned_rows(oracle, cuda_device, O):
+    from test_gpu_seq import run_seq
+    run_seq(oracle, 2, 24, 16, 3, 3, 2, O, seed=O, int_rescaler=0.5)
