@@ -535,8 +535,8 @@ __global__ __launch_bounds__(kSfThreads) void k_fill_seq_lds(
     const uint32_t half = lane / L, cl = lane % L;
     uint32_t *my_rows = rowtab + (wave * kSlots + half) * C;
     // a bucket's slices run side by side on one XCD (workgroup i runs on XCD
-    // i % 8), so that its 1 KiB rows are fetched whole (config-5 attention layer:
-    // 2.73 -> 2.63 ms, and 1.50 -> 1.38 ms at an eighth of its batch)
+    // i % 8), so that its 1 KiB rows are fetched whole (S = 256, T = 64, 65536
+    // rows a table, O = 256: 2.73 -> 2.63 ms at B = 32, 1.50 -> 1.38 at B = 4)
     uint32_t slice = blockIdx.x % n_slices, rank = blockIdx.x / n_slices;
     if (gridDim.x % (8u * n_slices) == 0) {
         const uint32_t local = blockIdx.x / 8u;
