@@ -2555,7 +2555,7 @@ uint32_t seq_fill_cols(const SeqShape &s) {
 // The forward reads rows where they are (k_fill_seq_rows) rather than staging
 // every (table, Q) sub-table in LDS while the causal pairs select a table's rows
 // up to three times on average.  T = 64, 65536 rows a table, O = 256, S = 256, rows
-// against staging: 350 / 1210 us at half a pair a row, 1010 / 1380 at two, 1400 /
+// against staging: 335 / 1210 us at half a pair a row, 930 / 1380 at two, 1245 /
 // 1440 at three, 1680 / 1480 at four, 3630 / 2630 at sixteen.  Rows too where the
 // staging does not apply (odd widths: B = 32, 16384 rows, O = 255: 3170 us, 17360
 // with a wavefront an output row, k_fill_seq).
@@ -2564,6 +2564,21 @@ bool seq_fill_by_rows(const SeqShape &s) {
     if (!seq_partials_fit(s) || sub_rows * s.n_outputs * 4 > 0x7fffffffull) return false;
     const uint64_t pairs = (uint64_t)s.batch * s.seq * (s.seq - 1) / 2;
     return pairs <= 3 * (sub_rows << s.n_anchors) || seq_fill_cols(s) == 0;
+}
+
+// Wavefronts held back in k_fill_seq_rows: 12 a CU instead of 32, by LDS a workgroup
+// asks for and does not use (three workgroups of four a CU).  Past the 256 MB cache,
+// with few pairs a row, the second item that reads a row finds it cached only if the
+// items in flight leave it there: 32 wavefronts a CU stream through 512 MB of
+// sub-tables at once.  T = 64, 65536 rows a table, O = 256, S = 256: B = 4 1010 -> 930
+// us, B = 6 1420 -> 1245, B = 1 350 -> 335.  Not with many pairs a row (B = 32, 16384
+// rows, O = 255: 3140 -> 3530), small tables (16 of 4096 rows: 36 -> 39) or rows that
+// share a wavefront (O = 128: 551 -> 565).
+constexpr size_t kRowsHoldLds = 52 * 1024;
+bool seq_rows_hold(const SeqShape &s) {
+    const uint64_t table_rows = 1ull << (2 * s.n_anchors + s.pe_dim);
+    return s.n_detectors * table_rows * s.n_outputs * 4 > (256ull << 20) &&
+           (uint64_t)s.batch * s.seq * (s.seq - 1) / 2 <= 3 * table_rows;
 }
 
 // Columns of a weight-gradient slice (0: the sort path does not apply): a
@@ -2673,8 +2688,9 @@ hipError_t launch_forward_seq(const SeqShape &s, const float *w, const float *x,
         const uint32_t seg_units = ((rows + 7) / 8 + per_wg - 1) / per_wg;
         const uint64_t grid = 8ull * seg_units * n_slices * s.n_detectors;
         if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
+        const size_t hold = wide && seq_rows_hold(s) ? kRowsHoldLds : 0;
 #define SPIKY_FROWS(V, WD, IM)                                                                     \
-    hipLaunchKernelGGL((k_fill_seq_rows<V, WD, IM>), dim3((uint32_t)grid), dim3(kBlock), 0, st, w,  \
+    hipLaunchKernelGGL((k_fill_seq_rows<V, WD, IM>), dim3((uint32_t)grid), dim3(kBlock), hold, st, w, \
                        pack, ppack, samples, part, s.batch, s.seq, s.n_outputs, s.n_detectors,      \
                        s.n_anchors, s.pe_dim, lanes, n_slices, seg_units, int_rescaler)
         if (vec == 1) {

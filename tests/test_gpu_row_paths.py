@@ -141,6 +141,14 @@ def test_seq_forward_rows(oracle, cuda_device, B, S, T, Nc, Npe, O, int_rescaler
     run_seq(oracle, B, S, 20, T, Nc, Npe, O, seed=S + O, int_rescaler=int_rescaler, int_grad=True)
 
 
+# tables past the 256 MB cache, whose wavefronts are held back: a row a wavefront,
+# and an odd row over two
+@pytest.mark.parametrize("S,O", [(40, 256), (33, 261)])
+def test_seq_forward_rows_large_tables(oracle, cuda_device, S, O):
+    from test_gpu_seq import run_seq
+    run_seq(oracle, 1, S, 20, 5, 6, 4, O, seed=S + O, int_grad=True)
+
+
 # S, Npe, O: the grouped input gradient over rows padded to 64, 128 and 256
 # outputs and the weight gradient's unaligned 16-byte pieces: one output, a piece
 # and one more, a slice and one more, two slices less one, widths past 128 at few
