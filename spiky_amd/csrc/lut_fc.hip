@@ -1157,8 +1157,12 @@ constexpr uint32_t kRowSamples = 8;
 // Past 2^14 items the pushes go through du and the LDS scatter: global fp32 and
 // int32 atomics run at about 5 G/s here (B = 512, T = 1024, O = 256, int32:
 // 203 us with a pair of atomics an item), and a small call saves the launch.
+// Only while one wavefront holds a whole item (up to 64 blocks of outputs): du has
+// one word an item, and the wavefronts of a wider row each have a part of its term,
+// which they add with atomics.
 bool propagate_rows_scatters(const FcShape &s) {
-    return input_grad_scatter_applies(s) && (uint64_t)s.batch * s.n_detectors > (1u << 14);
+    return input_grad_scatter_applies(s) && (uint64_t)s.batch * s.n_detectors > (1u << 14) &&
+           s.n_outputs <= (uint32_t)(kWave * kRowBlock);
 }
 
 // k_propagate_rows reads a step's tables with 31-bit byte offsets, and forms

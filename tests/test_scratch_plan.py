@@ -153,6 +153,17 @@ def test_config3_sizes():
     assert walk(dm, "FORWARD", B) == T * B + (T // 32) * B * O * 4
 
 
+@pytest.mark.parametrize("int_rescaler", [None, 0.5])
+def test_input_gradient_words(int_rescaler):
+    """The gathered-row input gradient's du holds one word an item, so only rows
+    that one wavefront holds whole (2048 outputs) use it; the parts of a wider
+    row's term are added straight to the input gradient."""
+    B, T = 128, 132  # past 2^14 items
+    for O, words in ((2047, B * T), (2048, B * T), (2049, 0), (2052, 0), (4100, 0), (50257, 0)):
+        dm = manager(48, O, T, 2, int_rescaler=int_rescaler)
+        assert walk(dm, "BACKWARD_NO_WGRAD", B) == words * 4
+
+
 def test_allocation_free_limit():
     # the allocation-free forward's static array holds 64 MiB: the GPU test's
     # refused shape (B 8192) needs more, its accepted ones (1024, 300) less
