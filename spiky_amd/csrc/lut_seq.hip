@@ -381,11 +381,12 @@ __global__ __launch_bounds__(kBlock) void k_fill_seq_rows(
     }
     if (!on) return;
     uint32_t *dst = part + ((size_t)t * n_rows + row) * n_outputs + cs;
+    // position 0 has no pairs: its -0.0f leaves every accumulated output's bits as they are
     uint32_t o[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; v++)
         o[v] = INT_MODE ? (uint32_t)(int32_t)(acc[v] * kDenom32 * int_rescaler)
-                        : __float_as_uint((float)acc[v]);
+                        : __float_as_uint(j > 0 ? (float)acc[v] : -0.0f);
     if constexpr (VEC == 4)
         __builtin_nontemporal_store(u32x4u{o[0], o[1], o[2], o[3]}, reinterpret_cast<u32x4u *>(dst));
     else

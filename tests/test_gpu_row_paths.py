@@ -143,6 +143,35 @@ def test_seq_forward_rows(oracle, cuda_device, B, S, T, Nc, Npe, O, int_rescaler
     run_seq(oracle, B, S, 20, T, Nc, Npe, O, seed=S + O, int_rescaler=int_rescaler, int_grad=True)
 
 
+# B, S, T, Nc, Npe, O: rows where they are (narrow, odd, a row a wavefront), staged slices
+@pytest.mark.parametrize("B,S,T,Nc,Npe,O", [(2, 9, 5, 4, 2, 8), (1, 12, 40, 3, 1, 33), (2, 20, 7, 4, 2, 256),
+                                            (3, 20, 30, 3, 0, 261), (6, 40, 8, 2, 1, 64)])
+def test_seq_forward_first_position(oracle, cuda_device, B, S, T, Nc, Npe, O):
+    """Position 0 has no pairs: what its outputs hold stays, bit for bit
+    (negative zeros); every other position is added to."""
+    from test_gpu_seq import make_seq_dm, seq_inputs
+    x, anchors, W, pe, _ = seq_inputs(O, B, S, 20, T, Nc, Npe, O)
+    dm = make_seq_dm(20, O, T, Nc, S, Npe)
+    dev = torch.device("cuda:0")
+    before = torch.randn(B, S, O, generator=torch.Generator().manual_seed(4))
+    before[..., ::3] = -0.0
+    out = before.reshape(-1).to(dev)
+    idx, mi = (torch.empty(B * S * T, dtype=torch.int32, device=dev) for _ in range(2))
+    pli, pmi = (torch.empty((S - 1) * T, dtype=torch.int32, device=dev) if Npe else None for _ in range(2))
+    md, pmd = torch.empty(B * S * T, device=dev), torch.empty((S - 1) * T, device=dev) if Npe else None
+    print(f"[seq] first position S={S} T={T} O={O}", flush=True)
+    dm.forward_step_concat(W.to(dev), B, x.to(dev), anchors.to(dev), out, idx, 0.0, pe.to(dev) if Npe else None,
+                           pli, md, mi, pmd, pmi)
+    got, before = out.cpu().view(B, S, O).numpy(), before.numpy()
+    assert np.array_equal(got[:, 0].copy().view(np.int32), before[:, 0].copy().view(np.int32))
+    ridx, _, _ = oracle.check_detectors(x.numpy(), anchors.numpy(), B * S, 20, T, Nc)
+    rpli = oracle.check_pe(pe.numpy(), S, T, Npe)[0] if Npe else None
+    add = oracle.fill_outputs_seq(W.numpy(), ridx, rpli, B, O, T, S, Nc, Npe).reshape(B, S, O)
+    # T fp32 additions from another start
+    bound = (T + 1) * 2.0 ** -24 * (np.abs(before) + np.abs(add) + T * 0.01 * S)
+    assert np.all(np.abs(got.astype(np.float64) - before - add) <= bound)
+
+
 # tables past the 256 MB cache, whose wavefronts are held back: a row a wavefront,
 # and an odd row over two
 @pytest.mark.parametrize("S,O", [(40, 256), (33, 261)])
