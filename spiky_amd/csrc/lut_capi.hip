@@ -83,6 +83,11 @@ struct DeviceBuffer {
         bytes = 0;
         device = -1;
     }
+    bool holds(size_t need) const {
+        int cur = 0;
+        check_hip(hipGetDevice(&cur), "hipGetDevice");
+        return need == 0 || (ptr && device == cur && bytes >= need);
+    }
     // Make sure at least `need` bytes exist on the current device.
     void *ensure(size_t need) {
         int cur = 0;
@@ -838,9 +843,18 @@ int spiky_lut_backward_backprop(spiky_lut_manager *m, float *weights, uint32_t b
         float *target = (ext >= 0.0f) ? weights : weight_grad;
         const bool overwrite = overwrite_weight_grad != 0 && target == weight_grad;
         if (m->fully_connected == 1) {
-            const FcBackwardRegions r = fc_backward_regions(m, s, target != nullptr);
+            FcBackwardRegions r = fc_backward_regions(m, s, target != nullptr);
             const bool tm = r.tm;
-            uint8_t *base = reinterpret_cast<uint8_t *>(m->scratch.ensure(r.prop_bytes + r.wg_bytes));
+            // An input gradient alone can do without scratch: a capture that would
+            // have to grow the buffer, which captures cannot, takes that form.
+            if (!tm && !target && !m->scratch.holds(r.prop_bytes)) {
+                hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+                check_hip(hipStreamIsCapturing(st, &cs), "hipStreamIsCapturing");
+                if (cs != hipStreamCaptureStatusNone) r.prop_bytes = 0;
+            }
+            uint8_t *base = r.prop_bytes + r.wg_bytes == 0
+                                ? nullptr
+                                : reinterpret_cast<uint8_t *>(m->scratch.ensure(r.prop_bytes + r.wg_bytes));
             const size_t cap = base ? m->scratch.bytes : 0;
             spiky::Scratch prop_scr = spiky::scratch_run(base, r.prop_bytes);
             spiky::Scratch wg_scr = spiky::scratch_run(base ? base + r.prop_bytes : nullptr, cap - r.prop_bytes);

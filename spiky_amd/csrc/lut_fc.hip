@@ -1246,13 +1246,15 @@ hipError_t launch_fill_fc_i8(const FcShape &s, const int8_t *q8, const float *sc
                     : launch_fill_fc<int8_t, false, true>(s, q8, scales, idx, out, int_rescaler, st);
 }
 
-// scratch: du [B][T] u32 for the scattered input gradient, else none
+// scratch: du [B][T] u32 for the scattered input gradient, else none; without a
+// buffer the pushes are direct
 hipError_t launch_propagate_fc(const FcShape &s, const float *w, const float *g,
                                const int32_t *idx, const float *min_deltas,
                                const int32_t *min_idx, const int32_t *anchors, float *x_grad,
                                bool int_mode, double int_rescaler, Scratch &scratch, hipStream_t st) {
     const bool rows = propagate_rows_applies(s, int_mode);
-    const bool scatter = rows && propagate_rows_scatters(s);
+    const bool direct = scratch.mode == Scratch::Run && scratch.ptr == nullptr;
+    const bool scatter = rows && !direct && propagate_rows_scatters(s);
     ScratchLayout lay(scratch);
     uint32_t *du = scatter ? lay.take<uint32_t>((size_t)s.batch * s.n_detectors * 4) : nullptr;
     hipError_t e;

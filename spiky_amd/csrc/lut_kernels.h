@@ -115,7 +115,7 @@ hipError_t launch_fill_fc_i8(const FcShape &s, const int8_t *q8, const float *sc
 
 // Min-margin input gradient; int_mode sums int32 payloads into x_grad's words
 // and leaves it converted to fp32.  Scratch: du [B][T] where the input gradient
-// is scattered from it.
+// is scattered from it; run without a buffer it is pushed directly.
 hipError_t launch_propagate_fc(const FcShape &s, const float *w, const float *g,
                                const int32_t *idx, const float *min_deltas,
                                const int32_t *min_idx, const int32_t *anchors, float *x_grad,

@@ -24,6 +24,35 @@ def test_propagate_rows(oracle, cuda_device, B, T, Nc, O, int_rescaler):
     run_fc(oracle, B, 48, T, Nc, O, seed=B + O, int_rescaler=int_rescaler)
 
 
+def test_input_gradient_in_a_first_capture(cuda_device):
+    """An input gradient without a weight gradient is captured by a manager that
+    has no scratch yet, and every replay gives the eager (scattered) call's."""
+    B, I, T, Nc, O = 64, 512, 2048, 9, 40
+    x, anchors, W, go = make_inputs(2, B, I, T, Nc, O)
+    dev = torch.device("cuda:0")
+    xd, ad, Wd, gd = (v.to(dev) for v in (x, anchors, W, go))
+    idx, mi = (torch.empty(B * T, dtype=torch.int32, device=dev) for _ in range(2))
+    md, out = torch.empty(B * T, device=dev), torch.zeros(B * O, device=dev)
+    first, other = (make_dm(I, O, T, Nc, int_rescaler=0.5) for _ in range(2))
+    for dm in (first, other):
+        dm.forward_step(Wd, B, xd, ad, out, idx, 0.0, None, md, mi)
+    want = torch.zeros(B * I, device=dev)
+    other.backward_backprop(Wd, B, gd, ad, idx, md, mi, want, -1.0, None, None)
+    xg = torch.zeros(B * I, device=dev)
+    torch.cuda.synchronize()
+    print("[capture] input gradient", flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        xg.zero_()
+        first.backward_backprop(Wd, B, gd, ad, idx, md, mi, xg, -1.0, None, None)
+    for rep in range(3):
+        xg.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        print(f"[capture] replay {rep}", flush=True)
+        assert torch.equal(xg, want)
+
+
 @pytest.mark.parametrize("O", [10, 33, 301])
 def test_rows_not_looked_up_are_not_read(oracle, cuda_device, O):
     """Rows that no sample selects hold NaN: a row whose last piece crosses into
