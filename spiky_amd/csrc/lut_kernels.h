@@ -84,6 +84,9 @@ constexpr double kEps = 0.00000000000000001;
 constexpr double kDenom32 = 1048575.0;
 constexpr double kDenom32Reciproc = 9.536752259018191e-07;
 
+// A launch's threads in one dimension, workgroups times their size, stay below 2^32.
+constexpr uint64_t kMaxLaunchThreads = 0xffffffffull;
+
 struct FcShape {
     uint32_t batch;
     uint32_t n_inputs;

@@ -40,6 +40,7 @@
 #include "lut_kernels.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -1385,7 +1386,8 @@ __global__ __launch_bounds__(kGrpThreads) void k_propagate_seq_grp(
     uint32_t gb, uint32_t per_xcd, uint32_t n_outputs) {
     constexpr uint32_t O = NCH * 32;
     using Dot = typename std::conditional<PAD, double, float>::type;
-    // the widest fp64 form has registers for one item's g: loaded when the item is taken
+    // the widest fp64 form holds one item's g, loaded when the item is taken (and spills
+    // 36 registers all the same)
     constexpr bool kOneSet = PAD && NCH == 8;
     constexpr uint32_t kRowBytes = O * 4;
     __shared__ __attribute__((aligned(16))) uint8_t tab[kGrpTabBytes];
@@ -2509,12 +2511,13 @@ uint64_t seq_tri_bytes(const SeqShape &s) {
     return (uint64_t)s.batch * s.n_detectors * ((uint64_t)s.seq * (s.seq - 1) / 2) * 8;
 }
 
-// The pair-parallel main pass and its triangle reduction apply (fp32 sums).
+// A per-table partial of the output, [T][B*S][O] words, stays within 8 GiB.
 bool seq_partials_fit(const SeqShape &s) {
     const uint64_t rows = (uint64_t)s.batch * s.seq;
     return rows <= 0x7fffffffull && (uint64_t)s.n_detectors * rows * s.n_outputs * 4 <= (8ull << 30);
 }
 
+// The pair-parallel main pass and its triangle reduction apply (fp32 sums).
 bool seq_pairs_applies(const SeqShape &s) {
     return s.n_outputs % 4 == 0 && s.n_outputs <= (uint32_t)kPairMaxO && seq_tri_bytes(s) <= (16ull << 30);
 }
@@ -2522,23 +2525,57 @@ bool seq_pairs_applies(const SeqShape &s) {
 // Outputs of the grouped input-gradient pass's rows in LDS: the next of 64, 128, 256.
 uint32_t seq_grp_width(const SeqShape &s) { return s.n_outputs <= 64 ? 64 : s.n_outputs <= 128 ? 128 : 256; }
 
+// Causal pairs of a table.
+uint64_t seq_pairs(const SeqShape &s) { return (uint64_t)s.batch * s.seq * (s.seq - 1) / 2; }
+
+// The grouped pass with padded rows is worth its launches and its staging of whole
+// tables.  Against the pair-parallel pass (whole quads) from 12 pairs a row, past 2 x
+// 10^5 pairs, once the buckets fill the chip (T = 64, us, pairs / grouped: O = 96, 4096
+// rows: 8 pairs a row 268 / 325, 32 814 / 670; 65536 rows: 2 a row 1134 / 1367, 16 7150 /
+// 4554; 2 x 10^6 pairs over 16 tables of 256 rows: 157 / 158, of 8 tables 752 / 935), wider than 128
+// outputs, where the padding is more, from 48 (O = 132, 64 a row: 2253 / 2293; 16 a
+// row, T = 64: 54 / 61).  Against one thread a pair and block (other widths) by both
+// times, as measured from 10^2 to 7 x 10^7 pairs over tables of 2^6 to 2^16 rows
+// (O = 33, T = 64, us, pairs / grouped: 4096 rows: 10^3 pairs a table 69 / 93, 10^4 327 / 175;
+// 65536 rows: 406 / 503, 3 x 10^4 1164 / 678; O = 1, T = 4 of 64 rows, 1.3 x 10^5: 154 / 398).
+bool seq_grp_pays(const SeqShape &s, int gb) {
+    const double pairs = (double)seq_pairs(s), rows = std::exp2(2 * s.n_anchors + s.pe_dim);
+    const double T = s.n_detectors, O = s.n_outputs, buckets = T * std::exp2(s.n_anchors);
+    if (s.n_outputs % 4 == 0 && s.n_outputs > 128) return pairs >= 48 * rows && buckets >= 1024;
+    if (s.n_outputs % 4 == 0) return pairs >= 12 * rows && pairs * T >= 2e5 && buckets >= 256;
+    const double width = seq_grp_width(s), groups = std::exp2((int)s.n_anchors - gb);
+    const double cached = std::min(1.0, T * rows * O * 4 / 256e6), blocks = std::ceil(O / s.ogs);
+    // a pair and block is a thread, and its pushes to one input or positional
+    // dimension queue up
+    const double queue = (s.seq - 1) * blocks * (s.pe_dim > 0 ? s.batch + 1.0 : 1.0);
+    const double pair_us =
+        23 + std::max(pairs * T * (1.6e-4 * blocks + O * (4.2e-6 + 1.2e-5 * cached)), 0.05 * queue);
+    const double work_us = T * s.batch * s.seq * groups * 7.7e-4 + pairs * T * (1.85e-5 + 4.15e-7 * width);
+    const double grp_us = 49 + T * rows * width * 4 * 3e-7 + work_us * 256 / std::min(256.0, buckets * groups);
+    return pair_us > 1.1 * grp_us;
+}
+
+// Every launch of the grouped pass holds its threads.
+bool seq_grp_launches(const SeqShape &s, int gb) {
+    const uint64_t rows = (uint64_t)s.batch * s.seq;
+    const uint64_t wgs = ((uint64_t)s.n_detectors << (2 * s.n_anchors - gb)) + 8;
+    return wgs * kGrpThreads <= kMaxLaunchThreads && (uint64_t)s.n_detectors * s.batch * kWave <= kMaxLaunchThreads &&
+           rows * s.n_detectors + kBlock <= kMaxLaunchThreads && rows * seq_grp_width(s) + kBlock <= kMaxLaunchThreads;
+}
+
 // K-group bits of the grouped input-gradient pass (-1: it does not apply):
-// the widest group whose 2^(gb + Npe) rows fit the 128 KiB LDS table.
+// the widest group whose 2^(gb + Npe) rows fit the 128 KiB LDS table.  Widths
+// that are not its own (64, 128, 256) come as padded rows where that pays.
 int seq_grp_bits(const SeqShape &s) {
     if (s.n_outputs > 256) return -1;
-    // padded rows: up to 128 outputs, odd widths (whose other form is one thread a pair
-    // and block: B = 32, T = 64, O = 255, 16384 rows a table: 214 -> 9 ms), and wider
-    // rows from 16 pairs a row (O = 252: 11.3 -> 9.3 ms with the weight gradient; at
-    // four pairs, B = 1, O = 200, 0.81 against 0.67 ms)
-    if (s.n_outputs > 128 && s.n_outputs != 256 && s.n_outputs % 4 == 0 &&
-        (uint64_t)s.batch * s.seq * (s.seq - 1) / 2 < 16ull << (2 * s.n_anchors + s.pe_dim))
-        return -1;
     if (s.n_anchors > 10 || s.seq < 2 || s.seq - 1 > (uint32_t)kGrpMaxDist) return -1;
     if ((uint64_t)s.batch * s.seq >= (1ull << 27)) return -1;  // rows in 27 bits of the item metadata
     uint32_t lr = 0;
     while ((kGrpTabBytes >> (lr + 1)) >= (int)(seq_grp_width(s) * 4)) lr++;
     if (s.pe_dim > lr) return -1;
-    return (int)std::min<uint32_t>(s.n_anchors, lr - s.pe_dim);
+    const int gb = (int)std::min<uint32_t>(s.n_anchors, lr - s.pe_dim);
+    if (seq_grp_width(s) != s.n_outputs && !(seq_grp_launches(s, gb) && seq_grp_pays(s, gb))) return -1;
+    return gb;
 }
 
 // Columns of a forward slice for k_fill_seq_lds (0: it does not apply): the
@@ -2578,8 +2615,7 @@ bool seq_fill_by_rows(const SeqShape &s) {
 constexpr size_t kRowsHoldLds = 52 * 1024;
 bool seq_rows_hold(const SeqShape &s) {
     const uint64_t table_rows = 1ull << (2 * s.n_anchors + s.pe_dim);
-    return s.n_detectors * table_rows * s.n_outputs * 4 > (256ull << 20) &&
-           (uint64_t)s.batch * s.seq * (s.seq - 1) / 2 <= 3 * table_rows;
+    return s.n_detectors * table_rows * s.n_outputs * 4 > (256ull << 20) && seq_pairs(s) <= 3 * table_rows;
 }
 
 // Columns of a weight-gradient slice (0: the sort path does not apply): a

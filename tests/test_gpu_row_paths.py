@@ -228,3 +228,15 @@ def test_seq_backward_padded_rows(oracle, cuda_device, B, S, Nc, Npe, O, policy)
 def test_seq_int32_unaligned_rows(oracle, cuda_device, O):
     from test_gpu_seq import run_seq
     run_seq(oracle, 2, 24, 16, 3, 3, 2, O, seed=O, int_rescaler=0.5)
+
+
+# B, S, T, Nc, Npe, O: enough pairs for the grouped input gradient over padded rows:
+# one output, a piece and one more, a slice less or more one, one output past 128, a
+# whole-quad width in each padded size, wide quads
+@pytest.mark.parametrize("B,S,T,Nc,Npe,O", [(4, 100, 40, 3, 0, 1), (4, 100, 40, 3, 1, 5), (3, 70, 33, 3, 2, 33),
+                                            (3, 60, 20, 4, 1, 65), (2, 66, 24, 3, 2, 127), (2, 50, 24, 3, 1, 129),
+                                            (2, 50, 24, 3, 1, 255), (1, 112, 33, 4, 1, 36), (1, 112, 33, 4, 1, 100),
+                                            (1, 80, 128, 3, 0, 132), (1, 80, 128, 3, 0, 252)])
+def test_seq_backward_grouped_padded_rows(oracle, cuda_device, B, S, T, Nc, Npe, O):
+    from test_gpu_seq import run_seq
+    run_seq(oracle, B, S, 24, T, Nc, Npe, O, seed=O)

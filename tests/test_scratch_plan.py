@@ -145,7 +145,6 @@ def test_config3_sizes():
     assert fwd == T * B + (T // 32 // 8) * B * O * 4
     bwd = walk(dm, "BACKWARD", B)
     prop = 3 * T * B * 4
-    align = lambda n: (n + 255) // 256 * 256
     assert bwd == prop + align(T * (E + 1) * 4) + align(T * B * 4) + B * O * 4
     assert fwd < 0.15e9 and bwd < 0.16e9
     # ordered sums keep one partial per 32-table block
@@ -162,6 +161,41 @@ def test_input_gradient_words(int_rescaler):
     for O, words in ((2047, B * T), (2048, B * T), (2049, 0), (2052, 0), (4100, 0), (50257, 0)):
         dm = manager(48, O, T, 2, int_rescaler=int_rescaler)
         assert walk(dm, "BACKWARD_NO_WGRAD", B) == words * 4
+
+
+def align(n):
+    return (n + 255) // 256 * 256
+
+
+def seq_backward_bytes(B, S, T, Nc, Npe, O):
+    """Bytes of the sequence backward's scratch without its form's own part, and
+    that part for each form (all regions at 256-byte boundaries)."""
+    rows, n_pe = B * S, (S - 1) * T
+    common = [rows * T * 8, n_pe * 8] + [rows * T * 8] * 3 + [n_pe * max(Npe, 1) * 8,
+              T * ((1 << Nc) + 1) * 4, T * rows * 4, rows * O * 4, rows * T * 4, T * ((2 << Nc) + 1) * 4,
+              T * rows * 4, T * (1 << Nc) * 4]
+    width = 64 if O <= 64 else 128 if O <= 128 else 256
+    lr = (131072 // (width * 4)).bit_length() - 1
+    groups = 1 << (Nc - min(Nc, lr - Npe))
+    own = {"pairs": [B * T * (S * (S - 1) // 2) * 8] * 2, "plain": [],
+           "grouped": ([rows * width * 4] if width != O else []) + [T * rows * 8] * 2 + [T * B * (groups + 1) * 4] * 2}
+    return {form: sum(align(n) for n in common + extra) for form, extra in own.items()}
+
+
+@pytest.mark.parametrize("B,S,T,Nc,Npe,O,form", [
+    # whole quads: the pair-parallel pass until a table's rows are used often
+    (1, 12, 8, 4, 0, 4, "pairs"), (4, 256, 64, 6, 4, 96, "pairs"), (32, 256, 64, 5, 2, 96, "grouped"),
+    (32, 256, 64, 6, 4, 60, "grouped"), (32, 256, 8, 4, 0, 60, "pairs"), (1, 46, 64, 2, 2, 132, "pairs"),
+    (32, 256, 64, 5, 4, 252, "grouped"),
+    # other widths: one thread a pair and block until its time is the larger
+    (1, 12, 64, 6, 4, 255, "plain"), (1, 46, 64, 5, 2, 33, "plain"), (1, 256, 8, 4, 0, 33, "grouped"),
+    (1, 256, 4, 2, 2, 1, "plain"), (32, 256, 64, 6, 4, 201, "grouped"), (1, 142, 64, 5, 2, 127, "grouped"),
+    # the pass's own widths: always
+    (1, 12, 8, 6, 4, 64, "grouped"), (1, 12, 8, 6, 4, 128, "grouped"), (1, 2, 1, 6, 4, 256, "grouped")])
+def test_seq_backward_forms(B, S, T, Nc, Npe, O, form):
+    need = walk(manager(24, O, T, Nc, S=S, Npe=Npe), "BACKWARD_CONCAT", B)
+    sizes = seq_backward_bytes(B, S, T, Nc, Npe, O)
+    assert abs(need - sizes[form]) < 256, {f: need - n for f, n in sizes.items()}
 
 
 def test_allocation_free_limit():
