@@ -20,7 +20,7 @@
 //   k_fill_seq_lds      the same with the (table, Q) sub-table's column slice in
 //                       LDS, for many pairs a row.
 //   k_fill_seq          the same with the tables walked by the wavefront itself,
-//                       where the partials would not fit.
+//                       where the partials would not fit and for a few short walks.
 //   k_propagate_seq     fp32 summation: one wavefront per (sample, table, j); for
 //                       8 pairs at a time it reads the main, flipped and
 //                       PE-flipped rows, reduces the dots with a DPP
@@ -2590,25 +2590,57 @@ uint32_t seq_fill_cols(const SeqShape &s) {
     return cols;
 }
 
+// The launch of k_fill_seq_rows.
+struct SeqRowsLaunch {
+    uint32_t vec, n_slices, lanes, seg_units;
+    bool wide;
+    uint64_t grid;
+};
+
+SeqRowsLaunch seq_rows_launch(const SeqShape &s) {
+    SeqRowsLaunch r;
+    r.vec = s.n_outputs >= 4 ? 4 : 1;
+    const uint32_t pieces = (s.n_outputs + r.vec - 1) / r.vec;
+    r.n_slices = (pieces + kWave - 1) / kWave;
+    r.lanes = (pieces + r.n_slices - 1) / r.n_slices;
+    r.wide = r.lanes > kWave / 2;
+    const uint32_t per_wg = kWPB * (r.wide ? 1 : kWave / r.lanes);
+    const uint64_t rows = (uint64_t)s.batch * s.seq;
+    r.seg_units = (uint32_t)(((rows + 7) / 8 + per_wg - 1) / per_wg);
+    r.grid = 8ull * r.seg_units * r.n_slices * s.n_detectors;
+    return r;
+}
+
 // The forward reads rows where they are (k_fill_seq_rows) rather than staging
 // every (table, Q) sub-table in LDS while the causal pairs select a table's rows
 // up to three times on average.  T = 64, 65536 rows a table, O = 256, S = 256, rows
 // against staging: 335 / 1210 us at half a pair a row, 930 / 1380 at two, 1245 /
-// 1440 at three, 1680 / 1480 at four, 3630 / 2630 at sixteen.  Rows too where the
-// staging does not apply (odd widths: B = 32, 16384 rows, O = 255: 3170 us, 17360
-// with a wavefront an output row, k_fill_seq).
-bool seq_fill_by_rows(const SeqShape &s) {
+// 1440 at three, 1680 / 1480 at four, 3630 / 2630 at sixteen.  Narrow rows share
+// wavefronts, whose chain of pairs (about 0.05 us a position) must not be longer than
+// what staging the tables takes (B = 4, S = 256, 65536 rows a table, O = 4: T = 1 64 /
+// 42 us, T = 8 71 / 61, T = 64 1.3 times as fast as staging).
+//
+// Rows too where the staging does not apply (odd widths: B = 32, 16384 rows, O =
+// 255: 3170 us, 17360 with a wavefront an output row, k_fill_seq), but for a few short
+// walks, which are one launch there and four here (T = 8: S = 12 28 / 24 us, S = 46 28 /
+// 42; T = 1, S = 128 28 / 24; T = 16, S = 12 27 / 33).  There int32 sums take one more
+// launch a sample (B = 52, S = 34, T = 1, O = 127: 41 / 159).
+bool seq_fill_by_rows(const SeqShape &s, bool int_mode) {
     const uint64_t sub_rows = 1ull << (s.n_anchors + s.pe_dim);
     if (!seq_partials_fit(s) || sub_rows * s.n_outputs * 4 > 0x7fffffffull) return false;
-    const uint64_t pairs = (uint64_t)s.batch * s.seq * (s.seq - 1) / 2;
-    return pairs <= 3 * (sub_rows << s.n_anchors) || seq_fill_cols(s) == 0;
+    if (seq_rows_launch(s).grid * kBlock > kMaxLaunchThreads) return false;
+    if (seq_fill_cols(s) == 0) return (uint64_t)s.n_detectors * (s.seq + 16) >= 350 || (int_mode && s.batch > 4);
+    const uint64_t table_rows = sub_rows << s.n_anchors;
+    if (seq_pairs(s) > 3 * table_rows) return false;
+    // us: a wavefront's chain of pairs against the staged workgroups' launch, bytes and rounds
+    const double T = s.n_detectors, staged = T * table_rows * s.n_outputs * 4;
+    return s.n_outputs > 32 || 0.05 * s.seq <= 4 + staged * 2e-7 + T * std::exp2(s.n_anchors) * 0.012;
 }
 
-// Wavefronts held back in k_fill_seq_rows: 12 a CU instead of 32, by LDS a workgroup
-// asks for and does not use (three workgroups of four a CU).  Past the 256 MB cache,
-// with few pairs a row, the second item that reads a row finds it cached only if the
-// items in flight leave it there: 32 wavefronts a CU stream through 512 MB of
-// sub-tables at once.  T = 64, 65536 rows a table, O = 256, S = 256: B = 4 1010 -> 930
+// Wavefronts held back in k_fill_seq_rows: 12 a CU instead of the 16 that its 112
+// registers allow, by LDS a workgroup asks for and does not use (three workgroups of
+// four wavefronts a CU).  Past the 256 MB cache, with few pairs a row, the second item
+// that reads a row finds it cached only if the items in flight leave it there.  T = 64, 65536 rows a table, O = 256, S = 256: B = 4 1010 -> 930
 // us, B = 6 1420 -> 1245, B = 1 350 -> 335.  Not with many pairs a row (B = 32, 16384
 // rows, O = 255: 3140 -> 3530), small tables (16 of 4096 rows: 36 -> 39) or rows that
 // share a wavefront (O = 128: 551 -> 565).
@@ -2673,11 +2705,11 @@ hipError_t launch_forward_seq(const SeqShape &s, const float *w, const float *x,
                               float cmp_eps, bool int_mode, double int_rescaler, Scratch &scratch,
                               hipStream_t st) {
     const uint32_t rows = s.batch * s.seq;
-    const bool by_rows = seq_fill_by_rows(s);
+    const bool by_rows = seq_fill_by_rows(s, int_mode);
     const uint32_t fcols = by_rows ? 0 : seq_fill_cols(s);
-    // scratch: packed keys [T][B*S] | positional keys [T][S-1] | and for the
-    // LDS-sliced forward: bucket offsets [T][2^Nc+1] | samples [T][B*S] |
-    // per-table partials [T][B*S][O]
+    // scratch: packed keys [T][B*S] | positional keys [T][S-1] | and for the forms
+    // over buckets (rows in place, LDS slices): bucket offsets [T][2^Nc+1] | samples
+    // [T][B*S] | per-table partials [T][B*S][O] | LDS slices: the buckets' order
     ScratchLayout lay(scratch);
     uint2 *pack = lay.take<uint2>((size_t)rows * s.n_detectors * 8);
     uint2 *ppack = lay.take<uint2>((size_t)s.n_detectors * (s.seq - 1) * 8);
@@ -2687,7 +2719,7 @@ hipError_t launch_forward_seq(const SeqShape &s, const float *w, const float *x,
         offsets = lay.take<int32_t>((size_t)s.n_detectors * ((1u << s.n_anchors) + 1) * 4);
         samples = lay.take<int32_t>((size_t)s.n_detectors * rows * 4);
         part = lay.take<uint32_t>((size_t)s.n_detectors * rows * s.n_outputs * 4);
-        order = lay.take<uint32_t>((size_t)s.n_detectors * (1u << s.n_anchors) * 4);
+        if (fcols > 0) order = lay.take<uint32_t>((size_t)s.n_detectors * (1u << s.n_anchors) * 4);
     }
     hipError_t e;
     if (lay.stop(&e, "forward_step_concat")) return e;
@@ -2716,23 +2748,15 @@ hipError_t launch_forward_seq(const SeqShape &s, const float *w, const float *x,
         if (e != hipSuccess) return e;
     }
     if (by_rows) {
-        const uint32_t vec = s.n_outputs >= 4 ? 4 : 1;
-        const uint32_t pieces = (s.n_outputs + vec - 1) / vec;
-        const uint32_t n_slices = (pieces + kWave - 1) / kWave;
-        const uint32_t lanes = (pieces + n_slices - 1) / n_slices;
-        const bool wide = lanes > kWave / 2;
-        const uint32_t per_wg = kWPB * (wide ? 1 : kWave / lanes);
-        const uint32_t seg_units = ((rows + 7) / 8 + per_wg - 1) / per_wg;
-        const uint64_t grid = 8ull * seg_units * n_slices * s.n_detectors;
-        if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
-        const size_t hold = wide && seq_rows_hold(s) ? kRowsHoldLds : 0;
+        const SeqRowsLaunch r = seq_rows_launch(s);
+        const size_t hold = r.wide && seq_rows_hold(s) ? kRowsHoldLds : 0;
 #define SPIKY_FROWS(V, WD, IM)                                                                     \
-    hipLaunchKernelGGL((k_fill_seq_rows<V, WD, IM>), dim3((uint32_t)grid), dim3(kBlock), hold, st, w, \
+    hipLaunchKernelGGL((k_fill_seq_rows<V, WD, IM>), dim3((uint32_t)r.grid), dim3(kBlock), hold, st, w, \
                        pack, ppack, samples, part, s.batch, s.seq, s.n_outputs, s.n_detectors,      \
-                       s.n_anchors, s.pe_dim, lanes, n_slices, seg_units, int_rescaler)
-        if (vec == 1) {
+                       s.n_anchors, s.pe_dim, r.lanes, r.n_slices, r.seg_units, int_rescaler)
+        if (r.vec == 1) {
             if (int_mode) SPIKY_FROWS(1, false, true); else SPIKY_FROWS(1, false, false);
-        } else if (wide) {
+        } else if (r.wide) {
             if (int_mode) SPIKY_FROWS(4, true, true); else SPIKY_FROWS(4, true, false);
         } else {
             if (int_mode) SPIKY_FROWS(4, false, true); else SPIKY_FROWS(4, false, false);

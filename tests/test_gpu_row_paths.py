@@ -230,6 +230,21 @@ def test_seq_int32_unaligned_rows(oracle, cuda_device, O):
     run_seq(oracle, 2, 24, 16, 3, 3, 2, O, seed=O, int_rescaler=0.5)
 
 
+# B, S, T, Nc, Npe, O: enough tables for the rows to be read where they are also at
+# widths that have no staged form (see the shapes above)
+@pytest.mark.parametrize("int_rescaler", [None, 0.5])
+@pytest.mark.parametrize("B,S,T,Nc,Npe,O", [(1, 2, 20, 4, 2, 1), (3, 17, 11, 3, 3, 3), (2, 9, 15, 4, 0, 33),
+                                            (1, 33, 8, 4, 2, 261), (6, 5, 2, 3, 2, 35), (1, 66, 5, 4, 4, 131)])
+def test_seq_forward_rows_any_width(oracle, cuda_device, B, S, T, Nc, Npe, O, int_rescaler):
+    from test_gpu_seq import run_seq
+    run_seq(oracle, B, S, 20, T, Nc, Npe, O, seed=S + O, int_rescaler=int_rescaler, int_grad=True)
+
+
+def test_seq_forward_rows_large_tables_two_slices(oracle, cuda_device):
+    from test_gpu_seq import run_seq
+    run_seq(oracle, 1, 64, 20, 5, 6, 4, 261, seed=325, int_grad=True)
+
+
 # B, S, T, Nc, Npe, O: enough pairs for the grouped input gradient over padded rows:
 # one output, a piece and one more, a slice less or more one, one output past 128, a
 # whole-quad width in each padded size, wide quads

@@ -198,6 +198,22 @@ def test_seq_backward_forms(B, S, T, Nc, Npe, O, form):
     assert abs(need - sizes[form]) < 256, {f: need - n for f, n in sizes.items()}
 
 
+@pytest.mark.parametrize("B,S,T,Nc,Npe,O,int_rescaler,form", [
+    (1, 256, 64, 6, 4, 256, None, "rows"), (32, 256, 64, 6, 4, 256, None, "staged"),
+    # narrow rows: staged where a wavefront's chain of pairs is longer than that
+    (4, 256, 2, 6, 4, 4, None, "staged"), (1, 142, 64, 5, 2, 4, None, "rows"), (1, 24, 8, 6, 4, 4, None, "rows"),
+    # odd widths: a few short walks are one launch; int32 sums end in one a sample
+    (1, 12, 8, 6, 4, 33, None, "walk"), (1, 46, 8, 6, 4, 33, None, "rows"), (1, 12, 64, 6, 4, 33, None, "rows"),
+    (52, 34, 1, 3, 2, 127, None, "walk"), (52, 34, 1, 3, 2, 127, 0.5, "rows")])
+def test_seq_forward_forms(B, S, T, Nc, Npe, O, int_rescaler, form):
+    need = walk(manager(24, O, T, Nc, S=S, Npe=Npe, int_rescaler=int_rescaler), "FORWARD_CONCAT", B)
+    rows = B * S
+    common = [rows * T * 8, (S - 1) * T * 8]
+    buckets = [T * ((1 << Nc) + 1) * 4, T * rows * 4, T * rows * O * 4]
+    own = {"walk": [], "rows": buckets, "staged": buckets + [T * (1 << Nc) * 4]}[form]
+    assert abs(need - sum(align(n) for n in common + own)) < 256
+
+
 def test_allocation_free_limit():
     # the allocation-free forward's static array holds 64 MiB: the GPU test's
     # refused shape (B 8192) needs more, its accepted ones (1024, 300) less
