@@ -1339,9 +1339,13 @@ hipError_t launch_wgrad_fc(const FcShape &s, const float *g, const int32_t *idx,
         // us at 32, 1924 at 4); so do lists of a few samples among untouched rows.
         const bool walk = s.batch >= 4 * s.n_entries || (!overwrite && !int_mode);
         // int32 rows cost a conversion each: 8 (B = 256, T = 1024, O = 256: 57 us, 66 at 4).
-        // Fewer again where few tables would leave the grid short of 32 wavefronts a CU.
+        // Fewer again where few tables would leave the grid short of 32 wavefronts a CU,
+        // more where a launch could not hold the wavefronts.
         uint32_t rpw = std::min<uint32_t>(s.n_entries, walk ? 32 : int_mode ? 8 : 4);
-        while (rpw > 4 && (uint64_t)n_slices * s.n_detectors * (s.n_entries / rpw) < 8192) rpw /= 2;
+        auto waves = [&](uint32_t r) { return (uint64_t)n_slices * s.n_detectors * (s.n_entries / r); };
+        while (rpw > 4 && waves(rpw) < 8192) rpw /= 2;
+        while (rpw < std::min<uint32_t>(s.n_entries, 32) && (waves(rpw) + kWPB * n_slices) * kWave > kMaxLaunchThreads)
+            rpw *= 2;
         const uint64_t units = (uint64_t)s.n_detectors * (s.n_entries / rpw);
         const uint64_t grid = (uint64_t)n_slices * ((units + kWPB - 1) / kWPB);
         if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
