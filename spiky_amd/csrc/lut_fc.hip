@@ -1339,11 +1339,16 @@ hipError_t launch_wgrad_fc(const FcShape &s, const float *g, const int32_t *idx,
         // us at 32, 1924 at 4); so do lists of a few samples among untouched rows.
         const bool walk = s.batch >= 4 * s.n_entries || (!overwrite && !int_mode);
         // int32 rows cost a conversion each: 8 (B = 256, T = 1024, O = 256: 57 us, 66 at 4).
-        // Fewer again where few tables would leave the grid short of 32 wavefronts a CU,
-        // more where a launch could not hold the wavefronts.
-        uint32_t rpw = std::min<uint32_t>(s.n_entries, walk ? 32 : int_mode ? 8 : 4);
+        // Narrow rows are little to write, and a wavefront's start and its list cost
+        // more: 32 rows up to 32 outputs (B = 3, T = 7000, E = 128, O = 16: 71 us at 4,
+        // 39 at 32; B = 2, T = 2048, E = 1024: 145 and 70), 16 up to 64 (O = 64: 72 at 4,
+        // 61 at 16, 62 at 32; B = 64, T = 1000, E = 256: 38, 29 and 30).
+        const uint32_t most = s.n_outputs <= 32 || walk ? 32 : s.n_outputs <= 64 ? 16 : int_mode ? 8 : 4;
+        uint32_t rpw = std::min<uint32_t>(s.n_entries, most);
+        // Fewer again where few tables would leave the grid short of 32 wavefronts a
+        // CU (narrow rows: 16), more where a launch could not hold the wavefronts.
         auto waves = [&](uint32_t r) { return (uint64_t)n_slices * s.n_detectors * (s.n_entries / r); };
-        while (rpw > 4 && waves(rpw) < 8192) rpw /= 2;
+        while (rpw > 4 && waves(rpw) < (s.n_outputs <= 64 ? 4096 : 8192)) rpw /= 2;
         while (rpw < std::min<uint32_t>(s.n_entries, 32) && (waves(rpw) + kWPB * n_slices) * kWave > kMaxLaunchThreads)
             rpw *= 2;
         const uint64_t units = (uint64_t)s.n_detectors * (s.n_entries / rpw);
