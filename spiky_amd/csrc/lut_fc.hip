@@ -496,7 +496,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-template <bool INT_MODE, bool SCATTER, bool ODD>
+template <bool INT_MODE, bool SCATTER, bool ODD, bool BIG>
 __global__ __launch_bounds__(kWave) void k_propagate_rows(
     const float *__restrict__ w, const float *__restrict__ g, const int32_t *__restrict__ idx,
     const float *__restrict__ md, const int32_t *__restrict__ mi, const int2 *__restrict__ anchors,
@@ -505,20 +505,20 @@ __global__ __launch_bounds__(kWave) void k_propagate_rows(
     uint32_t n_obc, uint32_t nob, uint32_t ib, uint32_t it, bool cut_units, double int_rescaler) {
     __shared__ __attribute__((aligned(16))) u32x4 rows[2][kWave * kRowPieces];
     const uint32_t lane = threadIdx.x;
-    // all samples of a run of tables on one XCD (workgroup i runs on XCD i % 8)
-    const uint32_t per_run = (batch + ib - 1) / ib * n_obc;
-    uint32_t r, rest;
-    if (n_runs >= 8) {
+    // all samples of a run of tables and a chunk of outputs on one XCD (workgroup i
+    // runs on XCD i % 8)
+    const uint32_t groups = (batch + ib - 1) / ib, n_units = n_runs * n_obc;
+    uint32_t job, b0;
+    if (n_units >= 8) {
         const uint32_t local = blockIdx.x / 8u;
-        r = (local / per_run) * 8u + blockIdx.x % 8u;
-        rest = local % per_run;
+        job = (local / groups) * 8u + blockIdx.x % 8u;
+        b0 = local % groups * ib;
     } else {
-        r = blockIdx.x % n_runs;
-        rest = blockIdx.x / n_runs;
+        job = blockIdx.x % n_units;
+        b0 = blockIdx.x / n_units * ib;
     }
-    if (r >= n_runs) return;
-    const uint32_t obc = rest % n_obc;
-    const uint32_t b0 = rest / n_obc * ib;
+    if (job >= n_units) return;
+    const uint32_t r = job / n_obc, obc = job % n_obc;
     const uint32_t t0 = r * run, t1 = min(t0 + run, n_detectors);
     // item i is sample b0 + i % ib of the step's table i / ib
     const uint32_t item = lane / nob, ol = lane % nob;
@@ -593,7 +593,38 @@ __global__ __launch_bounds__(kWave) void k_propagate_rows(
         return k;
     };
     u32x4 stage[2][kRowPieces];
+    // BIG: rows by their place in w instead, loads that the row ends cut short
+    auto load_rows_far = [&](uint32_t tb, const Key &k) {
+        constexpr uint64_t kNone = ~0ull;
+        const bool used = k.flip >= 0 && (uint32_t)k.flip < n_anchors;
+        const uint32_t rm = (uint32_t)k.row & (n_entries - 1);
+        const uint64_t t_row = (uint64_t)(tb + ti) * n_entries;
+        const uint64_t om = used ? (t_row + rm) * n_outputs + c0 : kNone;
+        const uint64_t oa = used ? (t_row + (rm ^ (1u << k.flip))) * n_outputs + c0 : kNone;
+        auto piece_of = [&](uint64_t o, int i) {
+            u32x4 v = u32x4{0u, 0u, 0u, 0u};
+            if (o == kNone || past[i]) return v;
+            const uint32_t *p = reinterpret_cast<const uint32_t *>(w) + o + piece * 4u;
+            if (col[i] + 4u <= n_outputs) {
+                const i32x4u x = *reinterpret_cast<const i32x4u *>(p);
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[q] = (uint32_t)x[q];
+            } else {
+#pragma unroll
+                for (int q = 0; q < 3; q++)
+                    if (col[i] + q < n_outputs) v[q] = p[q];
+            }
+            return v;
+        };
+#pragma unroll
+        for (int i = 0; i < kRowPieces; i++) {
+            const int u = 8 * i + (int)(lane >> 3);
+            stage[0][i] = piece_of(__shfl((unsigned long long)om, u, kWave), i);
+            stage[1][i] = piece_of(__shfl((unsigned long long)oa, u, kWave), i);
+        }
+    };
     auto load_rows = [&](uint32_t tb, const Key &k) {
+        if constexpr (BIG) return load_rows_far(tb, k);
         const float *wb = w + (size_t)tb * n_entries * n_outputs;
         const uint64_t left = (uint64_t)(n_detectors - tb) * n_entries * row_bytes;
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -1154,25 +1185,56 @@ bool rowsum_applies(const FcShape &s) {
 // from as many lines of the [B][T] index arrays.
 constexpr uint32_t kRowSamples = 8;
 
-// Past 2^14 items the pushes go through du and the LDS scatter: global fp32 and
-// int32 atomics run at about 5 G/s here (B = 512, T = 1024, O = 256, int32:
-// 203 us with a pair of atomics an item), and a small call saves the launch.
-// Only while one wavefront holds a whole item (up to 64 blocks of outputs): du has
-// one word an item, and the wavefronts of a wider row each have a part of its term,
-// which they add with atomics.
-bool propagate_rows_scatters(const FcShape &s) {
-    return input_grad_scatter_applies(s) && (uint64_t)s.batch * s.n_detectors > (1u << 14) &&
-           s.n_outputs <= (uint32_t)(kWave * kRowBlock);
-}
+// The launch of k_propagate_rows: its split of the work, or that it has none.
+struct RowsLaunch {
+    bool applies = false;
+    bool scatter = false;  // through du and the LDS scatter
+    bool big = false;      // tables past 31-bit byte offsets
+    uint32_t nob, n_obc, ib, it, run, n_runs, grid;
+};
 
-// k_propagate_rows reads a step's tables with 31-bit byte offsets, and forms
-// int32 payloads per 32 outputs.  A few thousand items of a block or less are one
-// wave's work of k_propagate_fc_exact on every CU, without the staging (B = 64,
-// T = 256, O = 10: 7.9 against 8.8 us).
-bool propagate_rows_applies(const FcShape &s, bool int_mode) {
-    if (s.n_outputs <= (uint32_t)kRowBlock && (uint64_t)s.batch * s.n_detectors <= (1u << 14)) return false;
-    if (int_mode && s.ogs != (uint32_t)kRowBlock) return false;
-    return (uint64_t)kWave * s.n_entries * std::max<uint32_t>(s.n_outputs, kRowBlock) * 4 < 0x7fffffffull;
+RowsLaunch rows_launch(const FcShape &s, bool int_mode) {
+    RowsLaunch r;
+    const uint64_t n_items = (uint64_t)s.batch * s.n_detectors;
+    if (int_mode && s.ogs != (uint32_t)kRowBlock) return r;  // payloads are formed per 32 outputs
+    // A few thousand items of a block or less are one wave's work of
+    // k_propagate_fc_exact on every CU, without the staging (B = 64, T = 256,
+    // O = 10: 7.9 against 8.8 us).
+    if (s.n_outputs <= (uint32_t)kRowBlock && n_items <= (1u << 14)) return r;
+    if (s.n_outputs >= (1u << 28)) return r;  // g's rows by 31-bit byte offsets
+    const uint32_t blocks = (s.n_outputs + kRowBlock - 1) / kRowBlock;
+    r.n_obc = (blocks + kWave - 1) / kWave;
+    r.nob = (blocks + r.n_obc - 1) / r.n_obc;
+    const uint32_t items = kWave / r.nob;
+    r.ib = std::min<uint32_t>({items, s.batch, kRowSamples});
+    // a step's tables are read by 31-bit byte offsets, by 64-bit ones from 2 GiB a table
+    const uint64_t table = (uint64_t)s.n_entries * std::max<uint32_t>(s.n_outputs, kRowBlock) * 4;
+    r.big = table > 0x7fffffffull;
+    r.it = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(items / r.ib, 0x7fffffffull / table));
+    // steps a wave: one until ~6144 waves (three rounds of 8 a CU) are in the grid, more
+    // where a launch could not hold the waves
+    const uint64_t groups = (s.batch + r.ib - 1) / r.ib;
+    const uint64_t steps = (s.n_detectors + r.it - 1) / r.it;
+    const uint64_t total = steps * groups * r.n_obc;
+    uint64_t per_wave = std::max<uint64_t>(1, std::min<uint64_t>(32, total / 6144));
+    for (;; per_wave *= 2) {
+        r.run = r.it * (uint32_t)std::min(per_wave, steps);
+        r.n_runs = (s.n_detectors + r.run - 1) / r.run;
+        const uint64_t units = (uint64_t)r.n_runs * r.n_obc;
+        const uint64_t grid = (units >= 8 ? (units + 7) / 8 * 8 : units) * groups;
+        r.grid = (uint32_t)grid;
+        if (grid * kWave <= kMaxLaunchThreads) break;
+        if (r.n_runs == 1) return r;
+    }
+    // Past 2^14 items the pushes go through du and the LDS scatter: global fp32 and
+    // int32 atomics run at about 5 G/s here (B = 512, T = 1024, O = 256, int32:
+    // 203 us with a pair of atomics an item), and a small call saves the launch.
+    // Only while one wavefront holds a whole item: du has one word an item, and the
+    // wavefronts of a row in chunks each have a part of its term, which they add with
+    // atomics.  At most 4 GiB of du.
+    r.scatter = r.n_obc == 1 && n_items > (1u << 14) && n_items <= (1u << 30) && input_grad_scatter_applies(s);
+    r.applies = true;
+    return r;
 }
 
 }  // namespace
@@ -1252,36 +1314,24 @@ hipError_t launch_propagate_fc(const FcShape &s, const float *w, const float *g,
                                const int32_t *idx, const float *min_deltas,
                                const int32_t *min_idx, const int32_t *anchors, float *x_grad,
                                bool int_mode, double int_rescaler, Scratch &scratch, hipStream_t st) {
-    const bool rows = propagate_rows_applies(s, int_mode);
-    const bool direct = scratch.mode == Scratch::Run && scratch.ptr == nullptr;
-    const bool scatter = rows && !direct && propagate_rows_scatters(s);
+    RowsLaunch r = rows_launch(s, int_mode);
+    if (scratch.mode == Scratch::Run && scratch.ptr == nullptr) r.scatter = false;
     ScratchLayout lay(scratch);
-    uint32_t *du = scatter ? lay.take<uint32_t>((size_t)s.batch * s.n_detectors * 4) : nullptr;
+    uint32_t *du = r.scatter ? lay.take<uint32_t>((size_t)s.batch * s.n_detectors * 4) : nullptr;
     hipError_t e;
     if (lay.stop(&e, "propagate_through_detectors_fc")) return e;
     const int2 *ap = reinterpret_cast<const int2 *>(anchors);
-    if (rows) {
-        const uint32_t blocks = (s.n_outputs + kRowBlock - 1) / kRowBlock;
-        const uint32_t n_obc = (blocks + kWave - 1) / kWave;
-        const uint32_t nob = (blocks + n_obc - 1) / n_obc;
-        const uint32_t items = kWave / nob;
-        const uint32_t ib = std::min<uint32_t>({items, s.batch, kRowSamples}), it = items / ib;
-        // steps a wave: one until ~6144 waves (three rounds of 8 a CU) are in the grid
-        const uint64_t groups = (uint64_t)((s.batch + ib - 1) / ib) * n_obc;
-        const uint64_t steps = (s.n_detectors + it - 1) / it * groups;
-        const uint64_t per_wave = std::min<uint64_t>(32, steps / 6144);
-        const uint32_t run = it * (uint32_t)std::max<uint64_t>(1, per_wave);
-        const uint32_t n_runs = (s.n_detectors + run - 1) / run;
-        const uint64_t grid = (uint64_t)(n_runs >= 8 ? (n_runs + 7) / 8 * 8 : n_runs) * groups;
-        if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
-#define SPIKY_PR(IM, SC, ODD)                                                                      \
-    hipLaunchKernelGGL((k_propagate_rows<IM, SC, ODD>), dim3((uint32_t)grid), dim3(kWave), 0, st, w, \
+    if (r.applies) {
+#define SPIKY_PR(IM, SC, ODD, BIG)                                                                 \
+    hipLaunchKernelGGL((k_propagate_rows<IM, SC, ODD, BIG>), dim3(r.grid), dim3(kWave), 0, st, w,    \
                        g, idx, min_deltas, min_idx, ap, x_grad, du, s.batch, s.n_inputs, s.n_outputs, \
-                       s.n_detectors, s.n_anchors, s.n_entries, run, n_runs, n_obc, nob, ib, it,    \
-                       s.ogs == (uint32_t)kRowBlock, int_rescaler)
+                       s.n_detectors, s.n_anchors, s.n_entries, r.run, r.n_runs, r.n_obc, r.nob, r.ib, \
+                       r.it, s.ogs == (uint32_t)kRowBlock, int_rescaler)
 #define SPIKY_PR_O(IM, SC)                                                                         \
-    if (s.n_outputs % 4 != 0) SPIKY_PR(IM, SC, true); else SPIKY_PR(IM, SC, false)
-        if (scatter) {
+    if (r.big) SPIKY_PR(IM, SC, true, true);                                                       \
+    else if (s.n_outputs % 4 != 0) SPIKY_PR(IM, SC, true, false);                                  \
+    else SPIKY_PR(IM, SC, false, false)
+        if (r.scatter) {
             if (int_mode) { SPIKY_PR_O(true, true); } else { SPIKY_PR_O(false, true); }
         } else {
             if (int_mode) { SPIKY_PR_O(true, false); } else { SPIKY_PR_O(false, false); }
@@ -1290,7 +1340,7 @@ hipError_t launch_propagate_fc(const FcShape &s, const float *w, const float *g,
 #undef SPIKY_PR
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        if (scatter) return launch_input_grad_scatter(s, du, min_idx, anchors, x_grad, int_mode, int_rescaler, st);
+        if (r.scatter) return launch_input_grad_scatter(s, du, min_idx, anchors, x_grad, int_mode, int_rescaler, st);
     } else {
         const uint32_t n_ob = (s.n_outputs + s.ogs - 1) / s.ogs;
         const uint64_t n_items = (uint64_t)s.batch * s.n_detectors * n_ob;

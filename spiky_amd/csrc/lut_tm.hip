@@ -1530,14 +1530,21 @@ static hipError_t launch_propagate_finish(const FcShape &s, float *dpart, uint32
                                      false, 1.0, st);
 }
 
-bool input_grad_scatter_applies(const FcShape &s) { return (uint64_t)s.n_inputs * 8 <= (uint64_t)kScatterLds; }
+// Samples a workgroup: as few as leaves a workgroup a CU, at most 16 or what LDS holds.
+static uint32_t scatter_samples(const FcShape &s) {
+    return std::max<uint32_t>(1, std::min<uint32_t>({16u, (uint32_t)kScatterLds / 8 / s.n_inputs, s.batch / 256}));
+}
+
+bool input_grad_scatter_applies(const FcShape &s) {
+    if ((uint64_t)s.n_inputs * 8 > (uint64_t)kScatterLds) return false;
+    const uint32_t spg = scatter_samples(s);
+    return ((uint64_t)s.batch + spg - 1) / spg * kScatterThreads <= kMaxLaunchThreads;
+}
 
 hipError_t launch_input_grad_scatter(const FcShape &s, const uint32_t *du, const int32_t *min_idx,
                                      const int32_t *anchors, float *x_grad, bool int_mode,
                                      double int_rescaler, hipStream_t st) {
-    // samples a workgroup: as few as leaves a workgroup a CU, at most 16 or what LDS holds
-    const uint32_t spg = std::max<uint32_t>(
-        1, std::min<uint32_t>({16u, (uint32_t)kScatterLds / 8 / s.n_inputs, s.batch / 256}));
+    const uint32_t spg = scatter_samples(s);
     const uint32_t groups = (s.batch + spg - 1) / spg;
     const bool small = (uint64_t)spg * s.n_inputs * 8 <= (uint64_t)kScatterLdsSmall;
 #define SPIKY_PS(IM, LDS)                                                                          \

@@ -37,3 +37,41 @@ def test_weight_gradient_rows(cuda_device):
         rows = idx.view(B, T)[b].long()
         want[torch.arange(T, device=dev), rows] += g[b]
     assert torch.equal(wg.view(T, E), want)
+
+
+def test_input_gradient_items(cuda_device):
+    """2^27 items of 32768 outputs, in 16 chunks: the gradients of some samples
+    against the same call over these samples alone, which one launch holds."""
+    B, I, T, Nc, O = 1 << 15, 2, 1 << 12, 1, 1 << 15
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(9)
+    g = torch.randn(B, O, device=dev, generator=gen)
+    W = torch.randn(T, 2, O, device=dev, generator=gen)
+    x = torch.randn(B * I, device=dev, generator=gen)
+    anchors = torch.tensor([0, 1], dtype=torch.int32, device=dev).repeat(T)
+    dm = make_dm(I, O, T, Nc)
+    idx, mi = (torch.empty(B * T, dtype=torch.int32, device=dev) for _ in range(2))
+    md = torch.empty(B * T, device=dev)
+    small = make_dm(I, 4, T, Nc)
+    small.forward_step(torch.zeros(T * 2 * 4, device=dev), B, x, anchors, torch.zeros(B * 4, device=dev), idx,
+                       0.0, None, md, mi)
+    some = [0, 1, 7, 8, 4095, B // 2 + 3, B - 1]
+    few = torch.tensor(some, device=dev)
+    pick = lambda v: v.view(B, T)[few].reshape(-1).contiguous()
+    dm.forward_step(W.view(-1), 1, x[:I].contiguous(), anchors, torch.zeros(O, device=dev),
+                    torch.empty(T, dtype=torch.int32, device=dev))
+    want = torch.zeros(len(some) * I, device=dev)
+    dm.backward_backprop(W.view(-1), len(some), g[few].reshape(-1), anchors, pick(idx), pick(md), pick(mi), want,
+                         -1.0, None, None)
+    xg = torch.zeros(B * I, device=dev)
+    print(f"[launch] input gradient B={B} T={T} O={O}", flush=True)
+    dm.backward_backprop(W.view(-1), B, g.view(-1), anchors, idx, md, mi, xg, -1.0, None, None)
+    got, want = xg.view(B, I)[few].double(), want.view(-1, I).double()
+    # fp32 additions of 16 T terms in any order: 16 T 2^-24 of the terms' magnitudes, that is
+    # the slope of at most 0.5 times the chunks' dots, which together are about four times
+    # the whole dot's
+    diff = (W[:, 1] - W[:, 0]).double()
+    exact = diff @ g[few].double().T  # [T][samples]
+    bound = 2 * 16 * T * 2.0 ** -24 * exact.abs().sum(0) + 1e-6 * want.abs().max(1).values
+    assert torch.all((got - want).abs().max(1).values <= bound)
+    assert torch.all(want.abs().max(1).values > 0)

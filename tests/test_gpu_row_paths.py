@@ -24,6 +24,43 @@ def test_propagate_rows(oracle, cuda_device, B, T, Nc, O, int_rescaler):
     run_fc(oracle, B, 48, T, Nc, O, seed=B + O, int_rescaler=int_rescaler)
 
 
+# B, T, Nc, O: as many tables a step as 31-bit offsets reach (all, one); tables of 2 GiB
+# and more, whose last row ends inside a piece or not
+@pytest.mark.parametrize("int_rescaler", [None, 0.5])
+@pytest.mark.parametrize("B,T,Nc,O", [(1, 70, 13, 1024), (1, 3, 19, 257), (5, 2, 15, 8190), (3, 1, 15, 16387),
+                                      (2, 1, 20, 516)])
+def test_propagate_large_tables(oracle, cuda_device, B, T, Nc, O, int_rescaler):
+    """Only the rows that the samples select are the same on both sides; the
+    oracle's other rows are never touched."""
+    I, E = 64, 1 << Nc
+    dev = torch.device("cuda:0")
+    x, anchors, _, go = make_inputs(3, B, I, T, Nc, 0)
+    go = torch.randn(B * O, generator=torch.Generator().manual_seed(O))
+    ridx, rmd, rmi = oracle.check_detectors(x.numpy(), anchors.numpy(), B, I, T, Nc)
+    Wd = torch.empty(T * E * O, device=dev).normal_(0.0, 0.01, generator=torch.Generator(device=dev).manual_seed(1))
+    W = np.zeros(T * E * O, np.float32)
+    for t in range(T):
+        for b in range(B):
+            row = ridx[b * T + t]
+            for r in (row, row ^ (1 << rmi[b * T + t])):
+                at = (t * E + r) * O
+                W[at:at + O] = Wd[at:at + O].cpu().numpy()
+    dm = make_dm(I, O, T, Nc, int_rescaler=int_rescaler)
+    idx, md, mi = (torch.from_numpy(v).to(dev) for v in (ridx, rmd, rmi))
+    out, xg = torch.zeros(B * O, device=dev), torch.zeros(B * I, device=dev)
+    print(f"[rows] large tables B={B} T={T} Nc={Nc} O={O} int={int_rescaler}", flush=True)
+    ad, gd = anchors.to(dev), go.to(dev)
+    dm.forward_step(Wd, B, x.to(dev), ad, out, idx, 0.0, None, md, mi)
+    dm.backward_backprop(Wd, B, gd, ad, idx, md, mi, xg, -1.0, None, None)
+    rxg = oracle.propagate_fc(W, go.numpy(), ridx, rmd, rmi, anchors.numpy(), B, I, O, T, Nc, E,
+                              int_mode=int_rescaler is not None, int_rescaler=int_rescaler or 1.0)
+    if int_rescaler is not None:
+        oracle.convert_int_to_float(rxg, int_rescaler)
+        assert np.array_equal(xg.cpu().numpy(), rxg)
+    else:
+        xg_close(xg.cpu().numpy(), rxg, B, I, T, (O + 31) // 32)
+
+
 def test_input_gradient_in_a_first_capture(cuda_device):
     """An input gradient without a weight gradient is captured by a manager that
     has no scratch yet, and every replay gives the eager (scattered) call's."""

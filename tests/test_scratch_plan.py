@@ -163,6 +163,13 @@ def test_input_gradient_words(int_rescaler):
         assert walk(dm, "BACKWARD_NO_WGRAD", B) == words * 4
 
 
+@pytest.mark.parametrize("Nc,O", [(12, 1024), (13, 1024), (14, 2047), (16, 200), (18, 2048)])
+def test_large_tables_keep_the_row_gradient(Nc, O):
+    """Up to tables of 2 GiB and past them: their input gradient is the gathered
+    rows' (whose scatter shows in the plan), however many tables a step spans."""
+    assert walk(manager(48, O, 2048, Nc), "BACKWARD_NO_WGRAD", 64) == 64 * 2048 * 4
+
+
 def align(n):
     return (n + 255) // 256 * 256
 
