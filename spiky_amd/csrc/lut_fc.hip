@@ -22,7 +22,8 @@
 //                       fp64 in output order (both summations).
 //   k_propagate_fc_exact one thread per (b, t, output block): the reference's
 //                       own decomposition, for int32 payloads of other block
-//                       sizes and for very small calls.
+//                       sizes, for few items of narrow rows and for rows of a
+//                       few outputs (see rows_launch).
 //   k_bucket_samples +  table-major weight gradient: a stable counting sort of
 //   k_wgrad_rowsum      the samples of every table by lookup index, then one
 //                       wavefront per table row summing g over its bucket in
@@ -1226,14 +1227,25 @@ RowsLaunch rows_launch(const FcShape &s, bool int_mode) {
         if (grid * kWave <= kMaxLaunchThreads) break;
         if (r.n_runs == 1) return r;
     }
-    // Past 2^14 items the pushes go through du and the LDS scatter: global fp32 and
-    // int32 atomics run at about 5 G/s here (B = 512, T = 1024, O = 256, int32:
-    // 203 us with a pair of atomics an item), and a small call saves the launch.
+    // Past 2^14 items the pushes go through du and the LDS scatter where that costs
+    // less than a pair of global atomics an item: about 0.1 us a thousand items, or
+    // 0.3 us an atomic on one input where few inputs take many (us, pushes / scatter;
+    // O = 64 unless said): B = 200, T = 2048: 48 / 28 with 512 inputs; B = 200, T = 512:
+    // 16 / 14; B = 16, T = 2048: 30 / 9 with 32 inputs; but B = 1200, T = 32, O = 12,
+    // 4096 inputs: 8 / 21; B = 2048, T = 128, O = 33, 12000 inputs: 32 / 69.
     // Only while one wavefront holds a whole item: du has one word an item, and the
     // wavefronts of a row in chunks each have a part of its term, which they add with
     // atomics.  At most 4 GiB of du.
-    r.scatter = r.n_obc == 1 && n_items > (1u << 14) && n_items <= (1u << 30) && input_grad_scatter_applies(s);
-    r.applies = true;
+    const double crowd_us = 0.6 * s.n_detectors / s.n_inputs;
+    const double scatter_us = input_grad_scatter_applies(s) ? input_grad_scatter_us(s, int_mode) : 1e30;
+    r.scatter = r.n_obc == 1 && n_items > (1u << 14) && n_items <= (1u << 30) &&
+                std::max(n_items * 95e-6, crowd_us) > scatter_us + 1.5;
+    // Rows of a few outputs are one thread's work an item: k_propagate_fc_exact, whose
+    // pushes take about 0.055 us a thousand, until the scatter saves more than the
+    // staging costs (O = 4, 512 inputs, exact / rows: B = 500, T = 128: 7 / 8 us; B =
+    // 64, T = 2048: 12 / 9; B = 200, T = 2048: 29 / 18).
+    r.applies = s.n_outputs > 8 || s.ogs < s.n_outputs ||
+                (r.scatter && std::max(n_items * 55e-6, crowd_us) > scatter_us + 4.0);
     return r;
 }
 

@@ -129,6 +129,11 @@ hipError_t launch_propagate_fc(const FcShape &s, const float *w, const float *g,
 // (x_grad is then converted to fp32).  0 marks no term.  Applies while a
 // sample's input row fits the LDS sums.
 bool input_grad_scatter_applies(const FcShape &s);
+// Its time in us, from its launch, what a sample's inputs (cleared, then added
+// to x_grad) and tables cost a workgroup, and the workgroups the chip holds at once;
+// int32 sums save the conversion of x_grad.  B = 2048, T = 8: 2, 16 and 48 us at
+// 512, 4096 and 12000 inputs; B = 16, T = 8192: 7 us at 512.
+double input_grad_scatter_us(const FcShape &s, bool int_mode);
 hipError_t launch_input_grad_scatter(const FcShape &s, const uint32_t *du, const int32_t *min_idx,
                                      const int32_t *anchors, float *x_grad, bool int_mode,
                                      double int_rescaler, hipStream_t st);

@@ -1541,12 +1541,25 @@ bool input_grad_scatter_applies(const FcShape &s) {
     return ((uint64_t)s.batch + spg - 1) / spg * kScatterThreads <= kMaxLaunchThreads;
 }
 
+static bool scatter_small(const FcShape &s) {
+    return (uint64_t)scatter_samples(s) * s.n_inputs * 8 <= (uint64_t)kScatterLdsSmall;
+}
+
+double input_grad_scatter_us(const FcShape &s, bool int_mode) {
+    const uint32_t spg = scatter_samples(s);
+    const uint32_t groups = (s.batch + spg - 1) / spg;
+    const uint32_t at_once = scatter_small(s) ? 512 : 256;
+    const double us = 2.5 + (double)((groups + at_once - 1) / at_once) * spg *
+                                (s.n_inputs * 0.0005 + s.n_detectors * 0.0006);
+    return int_mode ? us - 1.5 - (double)s.batch * s.n_inputs * 2e-6 : us;
+}
+
 hipError_t launch_input_grad_scatter(const FcShape &s, const uint32_t *du, const int32_t *min_idx,
                                      const int32_t *anchors, float *x_grad, bool int_mode,
                                      double int_rescaler, hipStream_t st) {
     const uint32_t spg = scatter_samples(s);
     const uint32_t groups = (s.batch + spg - 1) / spg;
-    const bool small = (uint64_t)spg * s.n_inputs * 8 <= (uint64_t)kScatterLdsSmall;
+    const bool small = scatter_small(s);
 #define SPIKY_PS(IM, LDS)                                                                          \
     hipLaunchKernelGGL((k_propagate_scatter<IM, LDS>), dim3(groups), dim3(kScatterThreads), 0, st,  \
                        du, min_idx, reinterpret_cast<const int2 *>(anchors), x_grad, s.batch,       \

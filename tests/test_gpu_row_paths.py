@@ -13,13 +13,13 @@ pytestmark = pytest.mark.gpu
 
 # B, T, Nc, O: a lone sample; one output; a block and one output more or less;
 # sample groups and tables that are not whole; more blocks than lanes (two
-# chunks); 512 rows a table; past the direct pushes (B * T > 2^14), also with rows of
-# two and three chunks, odd and even, and of exactly one
+# chunks); 512 rows a table; past the direct pushes (many tables on 48 inputs and B * T
+# > 2^14), also with rows of two and three chunks, odd and even, and of exactly one
 @pytest.mark.parametrize("int_rescaler", [None, 0.5])
 @pytest.mark.parametrize("B,T,Nc,O", [(1, 70, 4, 33), (1, 600, 3, 2), (9, 37, 5, 31), (7, 40, 4, 301),
                                       (3, 9, 2, 2049), (2, 5, 2, 4100), (17, 33, 9, 96),
-                                      (40, 430, 4, 63), (130, 130, 3, 5), (130, 130, 2, 2049),
-                                      (33, 520, 2, 4100), (130, 130, 2, 2048)])
+                                      (40, 430, 4, 63), (130, 130, 3, 5), (33, 520, 2, 2049),
+                                      (33, 520, 2, 4100), (33, 520, 2, 2048), (17, 1000, 3, 5), (33, 520, 4, 63)])
 def test_propagate_rows(oracle, cuda_device, B, T, Nc, O, int_rescaler):
     run_fc(oracle, B, 48, T, Nc, O, seed=B + O, int_rescaler=int_rescaler)
 

@@ -157,10 +157,28 @@ def test_input_gradient_words(int_rescaler):
     """The gathered-row input gradient's du holds one word an item, so only rows
     that one wavefront holds whole (2048 outputs) use it; the parts of a wider
     row's term are added straight to the input gradient."""
-    B, T = 128, 132  # past 2^14 items
+    B, T = 64, 4096
     for O, words in ((2047, B * T), (2048, B * T), (2049, 0), (2052, 0), (4100, 0), (50257, 0)):
         dm = manager(48, O, T, 2, int_rescaler=int_rescaler)
         assert walk(dm, "BACKWARD_NO_WGRAD", B) == words * 4
+
+
+@pytest.mark.parametrize("B,I,T,O,scatters", [
+    (64, 512, 2048, 64, True),           # many items of ordinary rows
+    (200, 512, 128, 64, False),          # 25600 items: two launches cost more than the pushes
+    (1200, 4096, 32, 100, False),        # few tables of many inputs: clearing them costs more
+    (2048, 12000, 128, 33, False),
+    (16, 32, 2048, 64, True),            # many pushes on few inputs
+    (64, 512, 512, 3, False),            # rows of a few outputs: one thread an item
+    (500, 512, 2048, 3, True),
+    (1 << 20, 512, 1024, 33, True),      # 4 GiB of du at most
+    (1 << 20, 512, 1025, 33, False),
+    ((1 << 26) - 16, 4, 1, 33, True),    # as many workgroups as a launch holds
+    (1 << 26, 4, 1, 33, False)])
+def test_input_gradient_scatter_rule(B, I, T, O, scatters):
+    dm = manager(I, O, T, 9)  # 512 rows a table: the gathered-row kernels at every batch
+    need = walk(dm, "BACKWARD_NO_WGRAD", B) if B * T * 4 % 256 == 0 else plan(dm, "BACKWARD_NO_WGRAD", B)[1]
+    assert need == ((B * T * 4 + 255) // 256 * 256 if scatters else 0)
 
 
 @pytest.mark.parametrize("Nc,O", [(12, 1024), (13, 1024), (14, 2047), (16, 200), (18, 2048)])
