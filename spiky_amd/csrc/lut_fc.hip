@@ -1205,6 +1205,13 @@ RowsLaunch rows_launch(const FcShape &s, bool int_mode) {
     if (s.n_outputs >= (1u << 28)) return r;  // g's rows by 31-bit byte offsets
     const uint32_t blocks = (s.n_outputs + kRowBlock - 1) / kRowBlock;
     r.n_obc = (blocks + kWave - 1) / kWave;
+    // Wide rows of many samples in up to eight chunks of 256 outputs or more, each an
+    // XCD's: its L2 then holds a chunk of the table that the samples are at, and the
+    // lanes of odd widths are filled (B = 1500, T = 64, E = 512: O = 1024 130 -> 77 us, O =
+    // 2048 235 -> 146; B = 150, T = 64, O = 1500 29 -> 15; at B = 64 the pushes of the
+    // parts cost more: int32, T = 64, E = 512, O = 1024 9 -> 12).
+    if (s.n_outputs >= 768 && s.batch >= 128)
+        r.n_obc = std::max<uint32_t>(r.n_obc, std::min<uint32_t>(8, (s.n_outputs + 255) / 256));
     r.nob = (blocks + r.n_obc - 1) / r.n_obc;
     const uint32_t items = kWave / r.nob;
     r.ib = std::min<uint32_t>({items, s.batch, kRowSamples});
@@ -1212,12 +1219,14 @@ RowsLaunch rows_launch(const FcShape &s, bool int_mode) {
     const uint64_t table = (uint64_t)s.n_entries * std::max<uint32_t>(s.n_outputs, kRowBlock) * 4;
     r.big = table > 0x7fffffffull;
     r.it = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(items / r.ib, 0x7fffffffull / table));
-    // steps a wave: one until ~6144 waves (three rounds of 8 a CU) are in the grid, more
-    // where a launch could not hold the waves
+    // steps a wave: one until ~6144 waves (three rounds of 8 a CU) are in the grid,
+    // a row in chunks up to eight, for which g is loaded once, from ~1536; more where a
+    // launch could not hold the waves
     const uint64_t groups = (s.batch + r.ib - 1) / r.ib;
     const uint64_t steps = (s.n_detectors + r.it - 1) / r.it;
     const uint64_t total = steps * groups * r.n_obc;
     uint64_t per_wave = std::max<uint64_t>(1, std::min<uint64_t>(32, total / 6144));
+    if (r.n_obc > 1) per_wave = std::max(per_wave, std::min<uint64_t>(8, total / 1536));
     for (;; per_wave *= 2) {
         r.run = r.it * (uint32_t)std::min(per_wave, steps);
         r.n_runs = (s.n_detectors + r.run - 1) / r.run;

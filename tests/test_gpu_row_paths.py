@@ -24,6 +24,13 @@ def test_propagate_rows(oracle, cuda_device, B, T, Nc, O, int_rescaler):
     run_fc(oracle, B, 48, T, Nc, O, seed=B + O, int_rescaler=int_rescaler)
 
 
+# B, T, Nc, O: wide rows of many samples in chunks (whole, odd, a lone block in the last)
+@pytest.mark.parametrize("int_rescaler", [None, 0.5])
+@pytest.mark.parametrize("B,T,Nc,O", [(128, 9, 3, 768), (131, 11, 3, 801), (130, 7, 5, 2048), (129, 5, 2, 2081)])
+def test_propagate_chunks(oracle, cuda_device, B, T, Nc, O, int_rescaler):
+    run_fc(oracle, B, 40, T, Nc, O, seed=B + O, int_rescaler=int_rescaler)
+
+
 # B, T, Nc, O: as many tables a step as 31-bit offsets reach (all, one); tables of 2 GiB
 # and more, whose last row ends inside a piece or not
 @pytest.mark.parametrize("int_rescaler", [None, 0.5])
