@@ -398,16 +398,24 @@ hipError_t launch_fill_blocks(const FcShape &s, const WT *w, const float *scales
     const uint32_t nq = (quads + n_slices - 1) / n_slices;
     n_slices = (quads + nq - 1) / nq;  // every slice starts inside the row
     const uint32_t n_blocks = (s.n_detectors + s.dgs - 1) / s.dgs;
-    const uint64_t grid = (uint64_t)n_slices * s.batch;
-    if (grid > 0x7fffffffu) return hipErrorInvalidConfiguration;
     const uint64_t want = std::max<uint64_t>((uint64_t)nq * n_blocks, nq * VEC);
     const uint32_t threads = (uint32_t)std::min<uint64_t>(kBlocksThreads, (want + kWave - 1) / kWave * kWave);
     const uint32_t width = nq * VEC + VEC;
     const uint32_t cap = std::min<uint32_t>(n_blocks, kBlocksLds / width);  // blocks of a chunk
-    hipLaunchKernelGGL((k_fill_blocks<WT, VEC, INT_MODE, SCALED>), dim3((uint32_t)grid), dim3(threads),
-                       cap * width * 4, st, w, scales, idx, out, s.n_outputs, s.n_detectors, s.n_entries,
-                       s.dgs, nq, n_slices, n_blocks, cap, int_rescaler);
-    return hipGetLastError();
+    // a launch holds fewer than 2^32 threads: more samples than that (4 M of 256
+    // columns with 1024 threads) take several
+    const uint32_t most = (uint32_t)std::max<uint64_t>(1, kMaxLaunchThreads / ((uint64_t)n_slices * threads));
+    for (uint32_t b0 = 0; b0 < s.batch;) {
+        const uint32_t nb = std::min(most, s.batch - b0);
+        hipLaunchKernelGGL((k_fill_blocks<WT, VEC, INT_MODE, SCALED>), dim3(n_slices * nb), dim3(threads),
+                           cap * width * 4, st, w, scales, idx + (size_t)b0 * s.n_detectors,
+                           out + (size_t)b0 * s.n_outputs, s.n_outputs, s.n_detectors, s.n_entries, s.dgs,
+                           nq, n_slices, n_blocks, cap, int_rescaler);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        b0 += nb;
+    }
+    return hipSuccess;
 }
 
 // ---------------------------------------------------------------------------

@@ -14,6 +14,32 @@ def anchors_of(T, Nc, I, dev, seed):
     return torch.stack([torch.randperm(I, generator=g)[:2] for _ in range(T * Nc)]).to(torch.int32).flatten().to(dev)
 
 
+@pytest.mark.parametrize("T", [1, 65])
+def test_forward_samples(cuda_device, T):
+    """One table and three blocks of tables (a workgroup a sample)."""
+    B, I, O, dgs = (1 << 26) + 77, 2, 1, 32
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(T)
+    x = torch.randn(B * I, device=dev, generator=gen)
+    W = torch.randn(T * 2, device=dev, generator=gen)
+    anchors = anchors_of(T, 1, I, dev, T)
+    out = torch.zeros(B, device=dev)
+    idx = torch.empty(B * T, dtype=torch.int32, device=dev)
+    print(f"[launch] forward B={B} T={T}", flush=True)
+    make_dm(I, O, T, 1, bgs=dgs).forward_step(W, B, x, anchors, out, idx)
+    a = anchors.view(T, 2).tolist()
+    want = torch.zeros(B, device=dev)
+    xs = x.view(B, I)
+    for t0 in range(0, T, dgs):
+        block = torch.zeros(B, dtype=torch.float64, device=dev)
+        for t in range(t0, min(t0 + dgs, T)):
+            bit = xs[:, a[t][0]] > xs[:, a[t][1]]
+            assert torch.equal(idx.view(B, T)[:, t].bool(), bit)
+            block += torch.where(bit, W[2 * t + 1], W[2 * t]).double()
+        want += block.float()
+    assert torch.equal(out, want)
+
+
 def test_weight_gradient_rows(cuda_device):
     """2^28 table rows."""
     B, I, T, Nc, O = 2, 32, 1 << 16, 12, 1
