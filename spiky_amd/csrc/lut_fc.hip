@@ -254,10 +254,18 @@ constexpr int kWPB = kBlock / kWave;  // wavefronts per workgroup
 //         B = 1024, T = 1024, E = 1024, O = 256:   244 -> 165 us
 //   int8  B = 32,   T = 4096, E = 256,  O = 1024:  399 -> 43 us
 //
+// Blocks smaller than the rows in flight are taken several at a time (RAGGED, up to
+// 16 tables, each block committed where it ends), and a unit's last rows four at a
+// time, so that few rows are loaded in vain: blocks of one table, B = 300, T = 512,
+// O = 256: 65 us, 240 with a block at a time, 185 walked; B = 1, T = 8192, O = 1024:
+// 152 and 214; blocks of 15 tables give up 10 % for it (B = 512, T = 256, O = 301:
+// 26.4 and 23.5).
+//
 // A quad that would cross the row's end starts at n_outputs - 4 instead: its
 // first columns repeat the quad before it, value for value.
 constexpr int kBlocksThreads = 1024;
-constexpr uint32_t kBlocksLds = 8448;  // most commit values in LDS (33 KiB): 234 blocks of 32 columns + 4
+constexpr int kBlocksTables = 16;      // rows in flight a thread
+constexpr uint32_t kBlocksLds = 8448;  // most commit values in LDS (33 KiB): 32 blocks of 256 columns + 4
 
 typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -276,13 +284,14 @@ __device__ __forceinline__ void load_columns(const WT *p, float *v) {
     }
 }
 
-template <typename WT, int VEC, bool INT_MODE, bool SCALED>
+template <typename WT, int VEC, bool INT_MODE, bool SCALED, bool RAGGED>
 __global__ __launch_bounds__(kBlocksThreads) void k_fill_blocks(
     const WT *__restrict__ w, const float *__restrict__ scales, const int32_t *__restrict__ idx,
     float *__restrict__ out, uint32_t n_outputs, uint32_t n_detectors, uint32_t n_entries,
-    uint32_t dgs, uint32_t nq, uint32_t n_slices, uint32_t n_blocks, uint32_t cap, double int_rescaler) {
+    uint32_t dgs, uint32_t bpu, uint32_t nq, uint32_t n_slices, uint32_t n_blocks, uint32_t cap,
+    double int_rescaler) {
     extern __shared__ uint32_t part[];  // a row of commit values for each block of a chunk
-    constexpr int U = 16;
+    constexpr int U = kBlocksTables;
     const uint32_t tid = threadIdx.x;
     const uint32_t slice = blockIdx.x % n_slices;
     const uint32_t b = blockIdx.x / n_slices;
@@ -323,36 +332,59 @@ __global__ __launch_bounds__(kBlocksThreads) void k_fill_blocks(
     }
     for (uint32_t k0 = 0; k0 < n_blocks; k0 += cap) {
         const uint32_t nk = min(cap, n_blocks - k0);
-        for (uint32_t k = g; on && k < nk; k += groups) {
-            const uint32_t t0 = (k0 + k) * dgs;
-            const uint32_t t1 = min(t0 + dgs, n_detectors);
+        for (uint32_t k = g * bpu; on && k < nk; k += groups * bpu) {
+            uint32_t *row = part + k * width + VEC + cs - c0;
             double acc[VEC];
+            auto commit = [&]() {
+#pragma unroll
+                for (int v = 0; v < VEC; v++) {
+                    row[v] = INT_MODE ? (uint32_t)(int32_t)(acc[v] * kDenom32 * int_rescaler)
+                                      : __float_as_uint((float)acc[v]);
+                    acc[v] = 0.0;
+                }
+                row += width;
+            };
+            const uint32_t t0 = (k0 + k) * dgs;
+            const uint32_t t1 = min(t0 + min(bpu, nk - k) * dgs, n_detectors);
+            uint32_t last = t0 + dgs - 1;  // table of the block at hand
 #pragma unroll
             for (int v = 0; v < VEC; v++) acc[v] = 0.0;
             for (uint32_t t = t0; t < t1; t += U) {
                 uint32_t r[U];
                 lookups(r, t);
                 float vals[U][VEC];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
+                auto load = [&](int u) {
                     const uint32_t tt = min(t + u, n_detectors - 1);
                     load_columns<WT, VEC>(wc + tt * table + (size_t)r[u] * n_outputs, vals[u]);
+                };
+                if (RAGGED) {
+                    // four rows at a time up to the unit's end
+#pragma unroll
+                    for (int u = 0; u < U; u += 4)
+                        if (t + u < t1) {
+#pragma unroll
+                            for (int i = 0; i < 4; i++) load(u + i);
+                        }
+                } else {
+#pragma unroll
+                    for (int u = 0; u < U; u++) load(u);
                 }
 #pragma unroll
                 for (int u = 0; u < U; u++) {
+                    if (RAGGED && t + u >= t1) break;
                     const float sc = SCALED ? scales[min(t + u, n_detectors - 1)] : 1.0f;
 #pragma unroll
                     for (int v = 0; v < VEC; v++) {
                         const float x = SCALED ? sc * vals[u][v] : vals[u][v];
-                        acc[v] += t + u < t1 ? (double)x : 0.0;
+                        acc[v] += (double)(t + u < t1 ? x : 0.0f);
+                    }
+                    if (RAGGED && (t + u == last || t + u + 1 == t1)) {
+                        commit();
+                        last += dgs;
                     }
                 }
             }
-            uint32_t *row = part + k * width + VEC + cs - c0;
-#pragma unroll
-            for (int v = 0; v < VEC; v++)
-                row[v] = INT_MODE ? (uint32_t)(int32_t)(acc[v] * kDenom32 * int_rescaler)
-                                  : __float_as_uint((float)acc[v]);
+            if (!RAGGED) commit();
         }
         __syncthreads();
         if (tid < nc) {
@@ -398,19 +430,26 @@ hipError_t launch_fill_blocks(const FcShape &s, const WT *w, const float *scales
     const uint32_t nq = (quads + n_slices - 1) / n_slices;
     n_slices = (quads + nq - 1) / nq;  // every slice starts inside the row
     const uint32_t n_blocks = (s.n_detectors + s.dgs - 1) / s.dgs;
-    const uint64_t want = std::max<uint64_t>((uint64_t)nq * n_blocks, nq * VEC);
-    const uint32_t threads = (uint32_t)std::min<uint64_t>(kBlocksThreads, (want + kWave - 1) / kWave * kWave);
+    // blocks a thread takes at a time; threads for those of a chunk
+    const uint32_t bpu = std::max<uint32_t>(1, kBlocksTables / s.dgs);
+    const bool ragged = s.dgs % kBlocksTables != 0;
     const uint32_t width = nq * VEC + VEC;
-    const uint32_t cap = std::min<uint32_t>(n_blocks, kBlocksLds / width);  // blocks of a chunk
+    const uint32_t cap = std::min<uint32_t>(n_blocks, kBlocksLds / width / bpu * bpu);  // blocks of a chunk
+    const uint32_t units = (cap + bpu - 1) / bpu;
+    const uint32_t want = std::max(nq * units, nq * VEC);
+    const uint32_t threads = std::min<uint32_t>(kBlocksThreads, (want + kWave - 1) / kWave * kWave);
     // a launch holds fewer than 2^32 threads: more samples than that (4 M of 256
     // columns with 1024 threads) take several
     const uint32_t most = (uint32_t)std::max<uint64_t>(1, kMaxLaunchThreads / ((uint64_t)n_slices * threads));
     for (uint32_t b0 = 0; b0 < s.batch;) {
         const uint32_t nb = std::min(most, s.batch - b0);
-        hipLaunchKernelGGL((k_fill_blocks<WT, VEC, INT_MODE, SCALED>), dim3(n_slices * nb), dim3(threads),
-                           cap * width * 4, st, w, scales, idx + (size_t)b0 * s.n_detectors,
-                           out + (size_t)b0 * s.n_outputs, s.n_outputs, s.n_detectors, s.n_entries, s.dgs,
-                           nq, n_slices, n_blocks, cap, int_rescaler);
+#define SPIKY_FB(RG)                                                                              \
+    hipLaunchKernelGGL((k_fill_blocks<WT, VEC, INT_MODE, SCALED, RG>), dim3(n_slices * nb), dim3(threads), \
+                       cap * width * 4, st, w, scales, idx + (size_t)b0 * s.n_detectors,           \
+                       out + (size_t)b0 * s.n_outputs, s.n_outputs, s.n_detectors, s.n_entries, s.dgs, \
+                       bpu, nq, n_slices, n_blocks, cap, int_rescaler)
+        if (ragged) SPIKY_FB(true); else SPIKY_FB(false);
+#undef SPIKY_FB
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         b0 += nb;
@@ -1319,9 +1358,13 @@ template <typename WT, bool INT_MODE, bool SCALED>
 static hipError_t launch_fill_fc(const FcShape &s, const WT *w, const float *scales, const int32_t *idx,
                                  float *out, double int_rescaler, hipStream_t st) {
     if ((uint64_t)s.batch * s.n_detectors * s.n_outputs == 0) return hipSuccess;
-    if (s.n_outputs >= 4 && (sizeof(WT) == 4 || s.n_outputs % 4 == 0))
-        return launch_fill_blocks<WT, 4, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st);
-    return launch_fill_blocks<WT, 1, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st);
+    const uint64_t n_blocks = (s.n_detectors + s.dgs - 1) / s.dgs;
+    const uint64_t outputs = (uint64_t)s.batch * s.n_outputs;
+    // four columns a thread once there is work for the chip (B = 16, O = 1024, T = 64: 7.5
+    // us, 6.5 with one; B = 200, O = 256, T = 300: 12.7 and 20.7)
+    return s.n_outputs >= 4 && (sizeof(WT) == 4 || s.n_outputs % 4 == 0) && outputs * n_blocks > (1u << 15)
+               ? launch_fill_blocks<WT, 4, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st)
+               : launch_fill_blocks<WT, 1, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st);
 }
 
 hipError_t launch_fill_fc_f32(const FcShape &s, const float *w, const int32_t *idx, float *out,
