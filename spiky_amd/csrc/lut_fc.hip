@@ -33,6 +33,7 @@
 #include "lut_kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace spiky {
 namespace {
@@ -188,54 +189,6 @@ __global__ __launch_bounds__(1024) void k_check_detectors_lds(
 // ---------------------------------------------------------------------------
 // fill_outputs_non_seq_fc_logic (proto:1214-1299), re-scheduled.
 // ---------------------------------------------------------------------------
-template <typename WT, int VEC>
-struct RowLoad;
-
-template <>
-struct RowLoad<float, 1> {
-    __device__ static void load(const float *p, float *v) { v[0] = p[0]; }
-};
-template <>
-struct RowLoad<float, 2> {
-    __device__ static void load(const float *p, float *v) {
-        const float2 q = *reinterpret_cast<const float2 *>(p);
-        v[0] = q.x;
-        v[1] = q.y;
-    }
-};
-template <>
-struct RowLoad<float, 4> {
-    __device__ static void load(const float *p, float *v) {
-        const float4 q = *reinterpret_cast<const float4 *>(p);
-        v[0] = q.x;
-        v[1] = q.y;
-        v[2] = q.z;
-        v[3] = q.w;
-    }
-};
-template <>
-struct RowLoad<int8_t, 1> {
-    __device__ static void load(const int8_t *p, float *v) { v[0] = (float)p[0]; }
-};
-template <>
-struct RowLoad<int8_t, 2> {
-    __device__ static void load(const int8_t *p, float *v) {
-        const char2 q = *reinterpret_cast<const char2 *>(p);
-        v[0] = (float)q.x;
-        v[1] = (float)q.y;
-    }
-};
-template <>
-struct RowLoad<int8_t, 4> {
-    __device__ static void load(const int8_t *p, float *v) {
-        const char4 q = *reinterpret_cast<const char4 *>(p);
-        v[0] = (float)q.x;
-        v[1] = (float)q.y;
-        v[2] = (float)q.z;
-        v[3] = (float)q.w;
-    }
-};
-
 constexpr int kWPB = kBlock / kWave;  // wavefronts per workgroup
 
 // Forward gather-sum.  A workgroup owns a sample's column slice, a thread VEC
@@ -270,17 +223,18 @@ constexpr uint32_t kBlocksLds = 8448;  // most commit values in LDS (33 KiB): 32
 typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
+typedef int8_t i8x4u __attribute__((ext_vector_type(4), aligned(1)));
+
 template <typename WT, int VEC>
 __device__ __forceinline__ void load_columns(const WT *p, float *v) {
-    if constexpr (VEC == 4 && sizeof(WT) == 4) {
-        const f32x4u q = *reinterpret_cast<const f32x4u *>(p);
+    if constexpr (VEC == 4) {
+        typedef typename std::conditional<sizeof(WT) == 1, i8x4u, f32x4u>::type Quad;
+        const Quad q = *reinterpret_cast<const Quad *>(p);
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = q[i];
-    } else if constexpr (VEC == 2 && sizeof(WT) == 4) {
-        v[0] = p[0];
-        v[1] = p[1];
+        for (int i = 0; i < 4; i++) v[i] = (float)q[i];
     } else {
-        RowLoad<WT, VEC>::load(p, v);
+#pragma unroll
+        for (int i = 0; i < VEC; i++) v[i] = (float)p[i];
     }
 }
 
@@ -1362,7 +1316,7 @@ static hipError_t launch_fill_fc(const FcShape &s, const WT *w, const float *sca
     const uint64_t outputs = (uint64_t)s.batch * s.n_outputs;
     // four columns a thread once there is work for the chip (B = 16, O = 1024, T = 64: 7.5
     // us, 6.5 with one; B = 200, O = 256, T = 300: 12.7 and 20.7)
-    return s.n_outputs >= 4 && (sizeof(WT) == 4 || s.n_outputs % 4 == 0) && outputs * n_blocks > (1u << 15)
+    return s.n_outputs >= 4 && outputs * n_blocks > (1u << 15)
                ? launch_fill_blocks<WT, 4, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st)
                : launch_fill_blocks<WT, 1, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st);
 }
