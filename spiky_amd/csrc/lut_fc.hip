@@ -16,6 +16,8 @@
 //                       ascending order through LDS -- the exact commit order
 //                       of the reference CPU path, so the output is
 //                       bit-identical to it.
+//   k_fill_walk         the same order with one wavefront per (few samples,
+//                       column slice), for a lone block or many outputs.
 //   k_propagate_rows    one wavefront per (few samples, run of tables); a lane
 //                       owns a 32-output block of a (sample, table) item, fed
 //                       from coalesced row reads through LDS, and sums it in
@@ -193,18 +195,15 @@ constexpr int kWPB = kBlock / kWave;  // wavefronts per workgroup
 
 // Forward gather-sum.  A workgroup owns a sample's column slice, a thread VEC
 // columns of one block of dgs tables at a time (16 rows in flight, fp64,
-// ascending tables); the blocks' commit values meet
-// in LDS and are added in ascending block order: the reference CPU path's
-// arithmetic and commit order, so the output is bit-identical to it, and no
-// scratch.  What bounds it is the gather (B = 128, T = 2048, E = 256, O = 1024:
-// 170 us, 1.1 GB of rows at 6.3 TB/s) and, for a lone sample, its few dependent
-// loads.  One wavefront a column slice walking all tables in order, which this
-// replaces, had 16 rows in flight a slice and paid a load latency for every 16
-// tables:
+// ascending tables); the blocks' commit values meet in LDS and are added in
+// ascending block order: the reference CPU path's arithmetic and commit order, so
+// the output is bit-identical to it, and no scratch.  What bounds it is the gather
+// (B = 128, T = 2048, E = 256, O = 1024: 166 us, 1.1 GB of rows at 6.5 TB/s) and, for
+// a lone sample, its few dependent loads.  Against one wavefront a column slice
+// walking all tables in order, with 16 rows in flight a slice (k_fill_walk):
 //   fp32  B = 1,    T = 8192, E = 256,  O = 1024:  532 -> 26 us
 //         B = 16,   T = 4096, E = 256,  O = 256:   255 -> 18 us
 //         B = 100,  T = 1000, E = 128,  O = 301:    72 -> 24 us
-//         B = 1024, T = 1024, E = 1024, O = 256:   244 -> 165 us
 //   int8  B = 32,   T = 4096, E = 256,  O = 1024:  399 -> 43 us
 //
 // Blocks smaller than the rows in flight are taken several at a time (RAGGED, up to
@@ -368,6 +367,116 @@ __global__ __launch_bounds__(kBlocksThreads) void k_fill_blocks(
     if (tid < nc)
         // convert_integers_to_floats_logic, proto:200-213
         *op = INT_MODE ? (float)(((double)irun * kDenom32Reciproc) / int_rescaler) : run;
+}
+
+// The same sums in order, a wavefront SPW samples' column slice: a lane walks all the
+// tables of its VEC columns, 16 rows in flight (32 with four samples), and adds a
+// block's commit value to the running output where the block ends: no LDS and no
+// barrier, but one chain of steps a wavefront.  It is for a lone block of tables, and
+// for as many outputs as fill the chip by themselves, where the gather bounds it
+// (B = 2048, T = 256, E = 512, O = 1024: 212 us, 289 with k_fill_blocks) and where
+// consecutive workgroups take consecutive column slices, so that up to eight of them
+// each keep to an XCD's L2 (O = 512, T = 64: 25 and 42 us).
+template <typename WT, int VEC, int SPW, bool INT_MODE, bool SCALED>
+__global__ __launch_bounds__(kBlock) void k_fill_walk(
+    const WT *__restrict__ w, const float *__restrict__ scales, const int32_t *__restrict__ idx,
+    float *__restrict__ out, uint32_t batch, uint32_t n_outputs, uint32_t n_detectors,
+    uint32_t n_entries, uint32_t dgs, uint32_t n_slices, double int_rescaler) {
+    constexpr uint32_t U = SPW == 1 ? 16 : 8;
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = uniform(threadIdx.x / kWave);
+    const uint32_t slice = blockIdx.x % n_slices;
+    const uint32_t b0 = (blockIdx.x / n_slices * kWPB + wave) * SPW;
+    if (b0 >= batch) return;
+    const uint32_t c = (slice * kWave + lane) * VEC;
+    const bool on = c < n_outputs;
+    const uint32_t cs = min(c, n_outputs - VEC);  // n_outputs >= VEC
+    const WT *wc = w + cs;
+    const size_t table = (size_t)n_entries * n_outputs;
+    // samples past the batch repeat the last one and are not stored
+    const int32_t *ib[SPW];
+#pragma unroll
+    for (int s = 0; s < SPW; s++) ib[s] = idx + (size_t)min(b0 + s, batch - 1) * n_detectors;
+
+    float run[SPW][VEC];
+    double acc[SPW][VEC];
+#pragma unroll
+    for (int s = 0; s < SPW; s++)
+#pragma unroll
+        for (int v = 0; v < VEC; v++) {
+            run[s][v] = out[(size_t)min(b0 + s, batch - 1) * n_outputs + cs + v];
+            acc[s][v] = 0.0;
+        }
+    uint32_t last = min(dgs, n_detectors) - 1;  // table of the block at hand
+    // N tables from t
+    auto step = [&](uint32_t t, auto n) {
+        constexpr uint32_t N = decltype(n)::value;
+        float vals[N][SPW][VEC];
+#pragma unroll
+        for (uint32_t u = 0; u < N; u++)
+#pragma unroll
+            for (int s = 0; s < SPW; s++) {
+                const uint32_t r = (uint32_t)ib[s][t + u] & (n_entries - 1);
+                load_columns<WT, VEC>(wc + (t + u) * table + (size_t)r * n_outputs, vals[u][s]);
+            }
+#pragma unroll
+        for (uint32_t u = 0; u < N; u++) {
+            const float sc = SCALED ? scales[t + u] : 1.0f;
+            const bool ends = t + u == last;
+#pragma unroll
+            for (int s = 0; s < SPW; s++)
+#pragma unroll
+                for (int v = 0; v < VEC; v++) acc[s][v] += (double)(SCALED ? sc * vals[u][s][v] : vals[u][s][v]);
+            if (!ends) continue;
+#pragma unroll
+            for (int s = 0; s < SPW; s++)
+#pragma unroll
+                for (int v = 0; v < VEC; v++) {
+                    if (INT_MODE)
+                        run[s][v] = __int_as_float(wrap_add(__float_as_int(run[s][v]),
+                                                            (int32_t)(acc[s][v] * kDenom32 * int_rescaler)));
+                    else
+                        run[s][v] += (float)acc[s][v];
+                    acc[s][v] = 0.0;
+                }
+            last = min(last + dgs, n_detectors - 1);
+        }
+    };
+    uint32_t t = 0;
+    for (; t + U <= n_detectors; t += U) step(t, std::integral_constant<uint32_t, U>());
+    for (; t + 4 <= n_detectors; t += 4) step(t, std::integral_constant<uint32_t, 4>());
+    for (; t < n_detectors; t++) step(t, std::integral_constant<uint32_t, 1>());
+    if (!on) return;
+#pragma unroll
+    for (int s = 0; s < SPW; s++) {
+        if (b0 + s >= batch) break;
+        float *ob = out + (size_t)(b0 + s) * n_outputs + cs;
+#pragma unroll
+        for (int v = 0; v < VEC; v++)
+            if (cs + v >= c)  // the columns before c are another lane's
+                ob[v] = INT_MODE ? (float)(((double)__float_as_int(run[s][v]) * kDenom32Reciproc) / int_rescaler)
+                                 : run[s][v];
+    }
+}
+
+template <typename WT, int VEC, int SPW, bool INT_MODE, bool SCALED>
+hipError_t launch_fill_walk(const FcShape &s, const WT *w, const float *scales, const int32_t *idx,
+                            float *out, double int_rescaler, hipStream_t st) {
+    const uint32_t n_slices = (s.n_outputs + kWave * VEC - 1) / (kWave * VEC);
+    // as many samples a launch as it can hold threads of
+    const uint64_t per_wg = kWPB * SPW;
+    const uint32_t most = (uint32_t)std::min<uint64_t>(s.batch, kMaxLaunchThreads / ((uint64_t)n_slices * kBlock) * per_wg);
+    for (uint32_t b0 = 0; b0 < s.batch;) {
+        const uint32_t nb = std::min(most, s.batch - b0);
+        const uint32_t grid = n_slices * (uint32_t)((nb + per_wg - 1) / per_wg);
+        hipLaunchKernelGGL((k_fill_walk<WT, VEC, SPW, INT_MODE, SCALED>), dim3(grid), dim3(kBlock), 0, st, w,
+                           scales, idx + (size_t)b0 * s.n_detectors, out + (size_t)b0 * s.n_outputs, nb,
+                           s.n_outputs, s.n_detectors, s.n_entries, s.dgs, n_slices, int_rescaler);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        b0 += nb;
+    }
+    return hipSuccess;
 }
 
 template <typename WT, int VEC, bool INT_MODE, bool SCALED>
@@ -1314,6 +1423,33 @@ static hipError_t launch_fill_fc(const FcShape &s, const WT *w, const float *sca
     if ((uint64_t)s.batch * s.n_detectors * s.n_outputs == 0) return hipSuccess;
     const uint64_t n_blocks = (s.n_detectors + s.dgs - 1) / s.dgs;
     const uint64_t outputs = (uint64_t)s.batch * s.n_outputs;
+#define SPIKY_FW(V, S) return launch_fill_walk<WT, V, S, INT_MODE, SCALED>(s, w, scales, idx, out, int_rescaler, st)
+    // Walked in order (us, E = 512, blocks of 32 tables, blocks / walked): one block
+    // (B = 255, O = 250, T = 19: 7.9 / 6.7), or enough outputs to fill the chip (O =
+    // 256, T = 128: B = 300 11 / 15, B = 600 18 / 18, B = 2048 45 / 31; O = 1024, T = 200,
+    // E = 64: B = 128 16 / 21, B = 255 33 / 29), if they are not so narrow that a wavefront is
+    // mostly idle (O = 33, B = 10000: T = 64 34 / 26, T = 200 39 / 56).  int8 rows are a
+    // quarter as long (B = 600, O = 512, T = 200: 26 / 33; B = 2500: 85 / 61).
+    // Tables that an L2 holds need more wavefronts (B = 1692, T = 1689, E = 4, O = 126: 104 / 146).
+    const uint64_t bytes = (uint64_t)s.n_detectors * s.n_entries * s.n_outputs * sizeof(WT);
+    const bool fills = sizeof(WT) == 1 ? outputs >= (1u << 19) && s.n_outputs >= 192
+                       : s.n_outputs >= 96 ? outputs >= (bytes <= (8u << 20) ? 6u << 16 : 3u << 16)
+                                           : outputs >= (1u << 18) && s.n_detectors <= 64;
+    if (n_blocks == 1 || fills) {
+        if (outputs <= (1u << 17) || s.n_outputs < 4) SPIKY_FW(1, 1);
+        if constexpr (sizeof(WT) == 4) {
+            // Four samples a wavefront, one column a lane while the tables are not much
+            // past the caches (B = 2048, O = 512: T = 64 25 us, 33 with four columns and
+            // 41 with one sample; T = 512 231, 222 and 283), else four columns (O = 2048, T = 256:
+            // 434, 599 with one column); a short walk of large tables has too few steps
+            // for it (B = 8192, O = 1024, E = 2048, T = 16: 96, 98 with one sample).
+            if (outputs < (1u << 20) && !(s.n_outputs < 96 && s.batch >= 4096)) SPIKY_FW(4, 1);
+            if (s.n_outputs <= 768 ? bytes <= (192ull << 20) : s.n_detectors < 32 && bytes <= (48ull << 20)) SPIKY_FW(1, 4);
+            if (s.n_detectors >= 32) SPIKY_FW(4, 4);
+        }
+        SPIKY_FW(4, 1);
+    }
+#undef SPIKY_FW
     // four columns a thread once there is work for the chip (B = 16, O = 1024, T = 64: 7.5
     // us, 6.5 with one; B = 200, O = 256, T = 300: 12.7 and 20.7)
     return s.n_outputs >= 4 && outputs * n_blocks > (1u << 15)

@@ -16,7 +16,7 @@ def anchors_of(T, Nc, I, dev, seed):
 
 @pytest.mark.parametrize("T", [1, 65])
 def test_forward_samples(cuda_device, T):
-    """One table and three blocks of tables (a workgroup a sample)."""
+    """One table (walked) and three blocks of tables (a workgroup a sample)."""
     B, I, O, dgs = (1 << 26) + 77, 2, 1, 32
     dev = torch.device("cuda:0")
     gen = torch.Generator(device=dev).manual_seed(T)

@@ -129,15 +129,7 @@ def test_rows_not_looked_up_are_not_read(oracle, cuda_device, O):
     xg_close(xg.cpu().numpy(), rxg, B, I, T, (O + 31) // 32)
 
 
-# B, T, Nc, O, dgs: fewer columns than a quad; a quad that crosses the row's end
-# in the first, a middle and the last slice; a lone block; a last block of one
-# table; block sizes around the 16 rows in flight; more blocks than a chunk of
-# LDS holds (O = 250: 33 blocks of 252 columns); 512 rows a table
-@pytest.mark.parametrize("ordered", [False, True])
-@pytest.mark.parametrize("B,T,Nc,O,dgs", [(1, 40, 3, 1, 32), (2, 33, 2, 3, 32), (3, 16, 4, 5, 32),
-                                          (70, 97, 3, 30, 32), (5, 64, 3, 259, 16), (300, 80, 3, 250, 2),
-                                          (9, 35, 9, 67, 17), (1, 300, 2, 1030, 1), (2, 5, 2, 4100, 32), (257, 12, 4, 6, 15)])
-def test_forward_blocks(oracle, cuda_device, B, T, Nc, O, dgs, ordered):
+def check_forward(oracle, B, T, Nc, O, dgs, ordered):
     """Bit-exact for fp32 and int32 sums and for int8 tables, with or without
     ordered sums."""
     I, E = 32, 1 << Nc
@@ -162,6 +154,31 @@ def test_forward_blocks(oracle, cuda_device, B, T, Nc, O, dgs, ordered):
                 oracle.convert_int_to_float(want, rescaler)
             assert np.array_equal(idx.cpu().numpy(), ridx)
             assert np.array_equal(out.cpu().numpy(), want)
+
+
+# B, T, Nc, O, dgs: fewer columns than a quad; a quad that crosses the row's end
+# in the first, a middle and the last slice; a lone block; a last block of one
+# table; block sizes around the 16 rows in flight; more blocks than a chunk of
+# LDS holds (O = 250: 33 blocks of 252 columns); 512 rows a table
+@pytest.mark.parametrize("ordered", [False, True])
+@pytest.mark.parametrize("B,T,Nc,O,dgs", [(1, 40, 3, 1, 32), (2, 33, 2, 3, 32), (3, 16, 4, 5, 32),
+                                          (70, 97, 3, 30, 32), (5, 64, 3, 259, 16), (300, 80, 3, 250, 2),
+                                          (9, 35, 9, 67, 17), (1, 300, 2, 1030, 1), (2, 5, 2, 4100, 32), (257, 12, 4, 6, 15)])
+def test_forward_blocks(oracle, cuda_device, B, T, Nc, O, dgs, ordered):
+    check_forward(oracle, B, T, Nc, O, dgs, ordered)
+
+
+# B, T, Nc, O, dgs: tables walked in order.  A lone block of one table and of 31, one
+# and four columns a lane; a quad over the row's end; one sample a wavefront over several
+# blocks (whole, ragged, one table each); four samples, the last wavefront's partly past
+# the batch, with one column a lane and with four; a short walk of large tables
+@pytest.mark.parametrize("ordered", [False, True])
+@pytest.mark.parametrize("B,T,Nc,O,dgs", [(1, 1, 3, 1, 32), (5, 31, 4, 67, 32), (300, 19, 3, 501, 32),
+                                          (70000, 5, 2, 2, 32), (400, 40, 3, 1030, 8), (401, 33, 3, 1030, 32),
+                                          (400, 13, 3, 999, 1), (2101, 22, 3, 501, 7), (4101, 10, 2, 65, 3),
+                                          (1102, 37, 3, 1001, 5), (830, 18, 10, 1301, 9)])
+def test_forward_walk(oracle, cuda_device, B, T, Nc, O, dgs, ordered):
+    check_forward(oracle, B, T, Nc, O, dgs, ordered)
 
 
 # B, T, Nc, O: rows of a lane, of a piece and of a slice and one output more or
