@@ -204,7 +204,8 @@ def test_weight_gradient_accumulates(oracle, cuda_device, O):
     free = np.ones((T, E), bool)
     for t in range(T):
         free[t, ridx.reshape(B, T)[:, t]] = False
-    before.view(T, E, O)[torch.from_numpy(free)][:, 1:2] = float("nan")
+    before.view(T, E, O)[..., 1][torch.from_numpy(free)] = float("nan")
+    assert torch.isnan(before).any()
     dm = make_dm(I, O, T, Nc)
     dev = torch.device("cuda:0")
     xd, ad, Wd, gd, wg = (v.to(dev) for v in (x, anchors, W, go, before))
@@ -289,6 +290,33 @@ def test_seq_backward_padded_rows(oracle, cuda_device, B, S, Nc, Npe, O, policy)
 def test_seq_int32_unaligned_rows(oracle, cuda_device, O):
     from test_gpu_seq import run_seq
     run_seq(oracle, 2, 24, 16, 3, 3, 2, O, seed=O, int_rescaler=0.5)
+
+
+@pytest.mark.parametrize("O", [64, 256])
+@pytest.mark.parametrize("overwrite", [True, False])
+def test_seq_gradient_target_alignment(oracle, cuda_device, O, overwrite):
+    """A weight gradient that starts 4 bytes past a 16-byte boundary gets the
+    aligned one's values."""
+    from test_gpu_seq import make_seq_dm, seq_inputs
+    B, S, I, T, Nc, Npe = 2, 30, 16, 3, 3, 2
+    x, anchors, W, pe, go = seq_inputs(6, B, S, I, T, Nc, Npe, O, int_grad=True)
+    dm = make_seq_dm(I, O, T, Nc, S, Npe)
+    dev = torch.device("cuda:0")
+    xd, ad, Wd, ped, gd = (v.to(dev) for v in (x, anchors, W, pe, go))
+    out = torch.zeros(B * S * O, device=dev)
+    idx, mi = (torch.empty(B * S * T, dtype=torch.int32, device=dev) for _ in range(2))
+    pli, pmi = (torch.empty((S - 1) * T, dtype=torch.int32, device=dev) for _ in range(2))
+    md, pmd = torch.empty(B * S * T, device=dev), torch.empty((S - 1) * T, device=dev)
+    dm.forward_step_concat(Wd, B, xd, ad, out, idx, 0.0, ped, pli, md, mi, pmd, pmi)
+    got = []
+    for shift in (0, 1):
+        wg = torch.ones(Wd.numel() + 1, device=dev)[shift:shift + Wd.numel()]
+        xg, peg = torch.zeros(B * S * I, device=dev), torch.zeros((S - 1) * T * Npe, device=dev)
+        print(f"[seq] gradient target O={O} shift={shift}", flush=True)
+        dm.backward_backprop_concat(Wd, B, gd, ad, idx, md, mi, xg, -1.0, pli, pmd, pmi, peg, wg,
+                                    overwrite_weights_gradients=overwrite)
+        got.append(wg.cpu().numpy())
+    assert np.array_equal(got[0], got[1])
 
 
 # B, S, T, Nc, Npe, O: enough tables for the rows to be read where they are also at
