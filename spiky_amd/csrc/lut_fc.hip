@@ -27,9 +27,9 @@
 //                       sizes, for few items of narrow rows and for rows of a
 //                       few outputs (see rows_launch).
 //   k_bucket_samples +  table-major weight gradient: a stable counting sort of
-//   k_wgrad_rowsum      the samples of every table by lookup index, then one
-//                       wavefront per table row summing g over its bucket in
-//                       ascending sample order (bit-identical to the reference
+//   k_wgrad_slices      the samples of every table by lookup index, then a
+//                       wavefront a few table rows, summing g over a row's bucket
+//                       in ascending sample order (bit-identical to the reference
 //                       CPU path) and writing the row once.  No HBM atomics, and
 //                       the caller's zero-fill of w_grad can be fused away.
 #include "lut_kernels.h"
