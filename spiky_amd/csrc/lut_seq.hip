@@ -2640,10 +2640,11 @@ bool seq_fill_by_rows(const SeqShape &s, bool int_mode) {
 // Wavefronts held back in k_fill_seq_rows: 12 a CU instead of the 16 that its 112
 // registers allow, by LDS a workgroup asks for and does not use (three workgroups of
 // four wavefronts a CU).  Past the 256 MB cache, with few pairs a row, the second item
-// that reads a row finds it cached only if the items in flight leave it there.  T = 64, 65536 rows a table, O = 256, S = 256: B = 4 1010 -> 930
-// us, B = 6 1420 -> 1245, B = 1 350 -> 335.  Not with many pairs a row (B = 32, 16384
-// rows, O = 255: 3140 -> 3530), small tables (16 of 4096 rows: 36 -> 39) or rows that
-// share a wavefront (O = 128: 551 -> 565).
+// that reads a row finds it cached only if the items in flight leave it there.  T = 64,
+// 65536 rows a table, O = 256, S = 256: B = 4 1010 -> 930 us, B = 6 1420 -> 1245, B = 1
+// 350 -> 335.  Not with many pairs a row (B = 32, 16384 rows, O = 255: 3140 -> 3530),
+// small tables (16 of 4096 rows: 36 -> 39) or rows that share a wavefront (O = 128: 551
+// -> 565).
 constexpr size_t kRowsHoldLds = 52 * 1024;
 bool seq_rows_hold(const SeqShape &s) {
     const uint64_t table_rows = 1ull << (2 * s.n_anchors + s.pe_dim);
